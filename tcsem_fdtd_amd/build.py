@@ -13,7 +13,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libtcsem.so")
 DRIVER = os.path.join(HERE, "tcsem_fdtd")
 ARCH = "gfx950"
-SOURCES = ["tcsem_host.cpp", "tcsem_kernels.hip", "tcsem_upcont.hip"]
+SOURCES = ["tcsem_host.cpp", "tcsem_kernels.hip", "tcsem_upcont.hip", "tcsem_upmat.hip"]
 
 # Packed-FP32 instructions are disabled for all device code of this project.
 HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result",

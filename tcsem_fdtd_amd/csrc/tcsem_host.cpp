@@ -440,6 +440,10 @@ struct tcsem_ctx {
   double *d_work = nullptr;
   int up_tiled = 0, MA = 0, MG = 0, XR = 0;
   long long sA = 0, sG = 0, sX = 0;
+  // the air boundary in matrix form (choose_air): tables and row operators, one allocation
+  int up_dense = 0;
+  char *d_dn = nullptr;
+  DenseOp dn{};
   double *d_scratch = nullptr;
   size_t scratch_bytes = 0;
   UpcontArgs<double> up64{};
@@ -781,6 +785,13 @@ UpcontArgs<T> upcont_args(tcsem_ctx *c) {
   p += c->gyT.size();
   double *w = c->d_work;
   u.tiled = c->up_tiled;
+  u.d = c->dn;
+  if (c->up_dense) {  // the matrix form's planes share the work buffer with the chain's
+    const long long ns = c->nslots;
+    u.d.P = w;
+    u.d.Rx = w + ns * c->dn.sP;
+    u.d.Ry = w + 2 * ns * c->dn.sP;
+  }
   if (c->up_tiled) {
     const long long ns = c->nslots;
     T *wt = (T *)w;  // tiled planes in the field type; complex entries are T pairs
@@ -794,7 +805,7 @@ UpcontArgs<T> upcont_args(tcsem_ctx *c) {
     u.tby = u.tbx + ns * c->sX;
     u.sX = c->sX;
     u.XR = c->XR;
-  } else {
+  } else if (!c->up_dense) {
     const long long ws = c->wstride * c->nslots;
     u.cplx = (double2 *)w;
     u.tx = w + 2 * ws;
@@ -872,8 +883,11 @@ int alloc_slots(tcsem_ctx *c, int nslots) {
   const size_t pb = (size_t)7 * nslots * c->pstride * c->esz;
   // bytes per slot: tiled chain A and G (complex of the field type) and Bx, By (field type);
   // line chain cplx (complex FP64), tx, bxr (also the y-padding rows), byr (FP64)
-  const size_t per_slot = c->up_tiled ? (size_t)(2 * c->sA + 2 * c->sG + 2 * c->sX) * c->esz
-                                      : (size_t)5 * c->wstride * sizeof(double);
+  // the matrix form 3 planes of 2 H x MP (FP64), beside the tiled chain's need (a model batch may run
+  // either), in place of the line chain's
+  const size_t chain = c->up_tiled ? (size_t)(2 * c->sA + 2 * c->sG + 2 * c->sX) * c->esz
+                                   : (c->up_dense ? 0 : (size_t)5 * c->wstride * sizeof(double));
+  const size_t per_slot = std::max(chain, (size_t)(3 * c->dn.sP) * sizeof(double));
   const size_t wb = (size_t)nslots * per_slot;
   if (hipMalloc(&c->d_fields, fb) != hipSuccess) return fail(TCSEM_ENOMEM, "field allocation of %zu bytes failed", fb);
   if (hipMalloc(&c->d_planes, pb) != hipSuccess) return fail(TCSEM_ENOMEM, "plane allocation failed");
@@ -2097,6 +2111,20 @@ int batch_records(tcsem_batch *b, int by, int pf, MarchArgs<T> &la, UpcontArgs<T
   la.k_hi = la.N - 1;
   la.k_lo = 1;
   ul.tiled = 1;
+  // the matrix form of the air boundary when every member has it (of one kind), else the tiled chain for all
+  {
+    ul.d = b->m[0]->dn;
+    bool have = true, always = false;
+    float kb = 0, w = 0, bm = 0;
+    for (const tcsem_ctx *c : b->m) {
+      have = have && c->dn.on && c->dn.kf32 == ul.d.kf32;
+      always = always || c->dn.on == 2;
+      kb += c->dn.kb;
+      w += c->dn.w;
+      bm += c->dn.bm;
+    }
+    ul.d.on = have && (always || dense_line(b->prec == 32, kb, w, bm)) ? 2 : 0;
+  }
   // the march's work list
   {
     std::vector<int> tiles(nm);
@@ -2793,6 +2821,113 @@ int tcsem_waveform(int ns, double sigma_t, double *t, double *dt, double *wave) 
   return waveform(ns, sigma_t, t, dt, wave);
 }
 
+extern "C++" {
+namespace {
+// Whether the matrix form of the air boundary is built (chain: TCSEM_UPCONT_CHAIN; "dense" and "fft" force it
+// on and off): 2 where it always runs -- beyond the tiled chain (working lengths over 2048) the line chain is
+// slower by an order of magnitude: 220 x 200 x 110 under 3914 x 3894, FP64, 60 steps: 481.8 ms / 22.3 ms --,
+// 1 where it runs for some number of slots (dense_pays).
+constexpr size_t kDenseMax = (size_t)16 << 30;  // row operators of one model
+int choose_air(tcsem_ctx *c, const char *chain) {
+  const HostGrid &g = c->g;
+  const tcsem_grid_info &I = g.info;
+  const int M = I.M, n3 = c->n3, aY = I.Any_New;
+  if (chain && std::strcmp(chain, "fft") == 0) return 0;
+  // the rows have to mirror about the middle of the plane (they do, up to rounding of the coordinates)
+  for (int j = 0; j < M; ++j)
+    if (std::fabs((g.Y[j] - g.Y[0]) - (g.Y[M - 1] - g.Y[M - 1 - j])) > 1e-9 * (g.Y[M - 1] - g.Y[0])) return 0;
+  for (int p = 0; p < aY; ++p)
+    for (int q = 0; q < n3; ++q)
+      if (std::fabs(c->wf[(size_t)p * n3 + q] - c->wb[(size_t)(aY - 1 - p) * n3 + n3 - 1 - q]) > 1e-9) return 0;
+  const size_t esz = c->up_tiled ? c->esz : 8;
+  const size_t bytes = (size_t)(I.L1 / 2 + 1) * M * (M + 1) * esz;
+  const size_t work = (size_t)3 * (I.L1 + 2) * (M + 32) * 8;
+  // the allocation-free entry point's work planes have to hold it where the tiled chain's fit them; LDS of
+  // k_dn_y at four slots
+  if (bytes > kDenseMax || (c->up_tiled && work > kUpcontScratchBytes) || M > 800) return 0;
+  if (!c->up_tiled || (chain && std::strcmp(chain, "dense") == 0)) return 2;
+  // point passes of the tiled chain: rows in and out along x, three transforms of each column, two working
+  // lengths each where Bluestein's
+  auto passes = [](const HostPlan &p) { return (p.m == p.n ? 1.0 : 2.0) * p.m * p.log2m; };
+  DenseOp &d = c->dn;
+  d.kb = (float)(bytes * 1e-6);
+  d.w = (float)((1.8 * M * passes(c->plx) + 3.0 * (I.L1 / 2 + 1) * passes(c->ply)) * 1e-6);
+  d.bm = (float)((double)I.L * M * I.N * 10.25 * c->esz * 1e-6);
+  const bool f = c->prec == 32;
+  return dense_line(f, d.kb, d.w, d.bm) || dense_line(f, d.kb, 32 * d.w, 32 * d.bm) ? 1 : 0;
+}
+
+// Builds the matrix form's operators on the device (c->dn, c->d_dn).
+int build_dense(tcsem_ctx *c) {
+  const tcsem_grid_info &I = c->g.info;
+  const int L = I.L, M = I.M, L1 = I.L1, M1 = I.M1, H = L1 / 2 + 1;
+  DenseOp &d = c->dn;
+  DenseBuild b{};
+  d.on = c->up_dense;
+  d.kf32 = c->up_tiled && c->prec == 32;
+  d.ldax = b.ldax = (2 * H + 31) / 32 * 32;
+  d.ldb = b.ldb = (L + 1 + 15) / 16 * 16;
+  d.MP = (M + 1 + 31) / 32 * 32;
+  d.sP = (long long)2 * H * d.MP;
+  const int ne = (M + 1) / 2, no = M / 2;
+  d.kstride = b.kstride = (long long)ne * (ne + (M + 1) / 2) + (long long)no * (no + M / 2 + 1);
+  b.Hy = M1 / 2 + 1;
+  b.ldy = (M / 2 + 1 + 31) / 32 * 32;
+  const size_t nax = (size_t)(L + 15) / 16 * 16 * d.ldax, nb = (size_t)(2 * H + 3) / 4 * 4 * d.ldb;
+  const size_t ntab = nax + 2 * nb + 2 * (size_t)(M / 2 + 1) + H;
+  const size_t kb = (size_t)H * d.kstride * (d.kf32 ? 4 : 8);
+  if (hipMalloc(&c->d_dn, ntab * 8 + kb) != hipSuccess)
+    return fail(TCSEM_ENOMEM, "air operators: %zu bytes", ntab * 8 + kb);
+  double *p = (double *)c->d_dn;
+  d.ax = b.ax = p;
+  d.bx = b.bx = p + nax;
+  d.by = b.by = b.bx + nb;
+  b.nt = b.by + nb;
+  b.ns = b.nt + (M / 2 + 1);
+  b.ng = b.ns + (M / 2 + 1);
+  d.nt = M1 % 2 == 0 ? b.nt : nullptr;
+  d.ns = b.ns;
+  d.ng = b.ng;
+  d.kop = b.kop = p + ntab;
+  const tcsem_setup &s = c->setup;
+  b.dzdx = s.dzmin / s.dxmin;
+  b.dzdy = s.dzmin / s.dymin;
+  b.rxy = s.dxmin / s.dymin;
+  b.ryx = s.dymin / s.dxmin;
+  std::vector<double> trig(2 * (size_t)L1 + 4 * (size_t)M1);
+  for (int q = 0; q < L1; ++q) {
+    trig[2 * q] = std::cos(2 * kPi * q / L1);
+    trig[2 * q + 1] = std::sin(2 * kPi * q / L1);
+  }
+  for (int q = 0; q < 2 * M1; ++q) {
+    trig[2 * (L1 + q)] = std::cos(kPi * q / M1);
+    trig[2 * (L1 + q) + 1] = std::sin(kPi * q / M1);
+  }
+  const size_t ny = (size_t)b.Hy * b.ldy, ng = (size_t)H * b.Hy, ntmp = trig.size() + 6 * ny + 2 * ng;
+  double *t = nullptr;
+  if (hipMalloc((void **)&t, ntmp * 8) != hipSuccess) return fail(TCSEM_ENOMEM, "air operator tables: %zu bytes", ntmp * 8);
+  b.tx = (const double2 *)t;
+  b.ty = b.tx + L1;
+  b.cw = t + trig.size();
+  b.sw = b.cw + ny;
+  b.cs = b.sw + ny;
+  b.ss = b.cs + ny;
+  b.ce = b.ss + ny;
+  b.se = b.ce + ny;
+  b.gx = b.se + ny;
+  b.gy = b.gx + ng;
+  hipError_t e = hipMemcpy(t, trig.data(), trig.size() * 8, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = launch_fill_zero(c->d_dn, ntab * 8, c->stream);
+  if (e == hipSuccess) e = launch_fill_zero(b.cw, (6 * ny + 2 * ng) * 8, c->stream);
+  if (e == hipSuccess) e = launch_dense_build(b, upcont_args<double>(c), d.kf32 != 0, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  (void)hipFree(t);
+  if (e != hipSuccess) return fail(TCSEM_EDEVICE, "air operators: %s", hipGetErrorString(e));
+  return TCSEM_OK;
+}
+}  // namespace
+}  // extern "C++"
+
 int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_ctx **out) {
   if (!s || !cond || !out) return fail(TCSEM_EINVAL, "null argument");
   if (precision != TCSEM_FP64 && precision != TCSEM_FP32) return fail(TCSEM_EINVAL, "precision must be 32 or 64");
@@ -2859,24 +2994,6 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
     spline_weights(c->n3, g.dy.data() + oy, g.Y.data() + oy, aY, g.Yn.data() + aY + Ny, idr.data(), c->wb);
     // wavenumber gains on the half spectrum (UpContinuation_gpu.cu:113-164)
     const int L1 = I.L1, M1 = I.M1, H = L1 / 2 + 1;
-    c->gx.assign((size_t)M1 * H, 0.0);
-    c->gy.assign((size_t)M1 * H, 0.0);
-    const double dzdx = s->dzmin / s->dxmin, dzdy = s->dzmin / s->dymin;
-    const double rxy = s->dxmin / s->dymin, ryx = s->dymin / s->dxmin;
-    for (int iy = 0; iy < M1; ++iy)
-      for (int ix = 0; ix < H; ++ix) {
-        const double v1 = (iy < M1 / 2 + 1) ? (1.0 * kPi * iy) / M1 * dzdy : -(1.0 * kPi * (M1 - iy)) / M1 * dzdy;
-        const double u1 = (1.0 * kPi * ix) / L1 * dzdx;
-        double gxv = 1.0, gyv = 1.0;
-        if (!(ix == 0 && iy == 0)) {
-          const double rr = u1 * u1 + v1 * v1;
-          const double upcc = std::exp(-std::sqrt(rr)) * (1.0 / std::sqrt(rr));
-          gxv = rxy * u1 * upcc;
-          gyv = ryx * v1 * upcc;
-        }
-        c->gx[(size_t)iy * H + ix] = gxv;
-        c->gy[(size_t)iy * H + ix] = gyv;
-      }
     make_plan(L1, c->plx);
     make_plan(M1, c->ply);
     // The tiled chain needs both working lengths <= 2048 (one wavefront per line, two LDS buffers)
@@ -2884,6 +3001,28 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
     const char *chain = std::getenv("TCSEM_UPCONT_CHAIN");
     const bool want_lines = chain && std::strcmp(chain, "lines") == 0;
     c->up_tiled = !want_lines && c->plx.m <= 2048 && c->ply.m <= 2048 && L <= c->plx.m + 2 && M <= c->ply.m + 2;
+    c->up_dense = !want_lines && choose_air(c, chain);
+    const bool chains = c->up_tiled || !c->up_dense;  // whether an FFT chain may run: its gains
+    if (chains) {
+      c->gx.assign((size_t)M1 * H, 0.0);
+      c->gy.assign((size_t)M1 * H, 0.0);
+      const double dzdx = s->dzmin / s->dxmin, dzdy = s->dzmin / s->dymin;
+      const double rxy = s->dxmin / s->dymin, ryx = s->dymin / s->dxmin;
+      for (int iy = 0; iy < M1; ++iy)
+        for (int ix = 0; ix < H; ++ix) {
+          const double v1 = (iy < M1 / 2 + 1) ? (1.0 * kPi * iy) / M1 * dzdy : -(1.0 * kPi * (M1 - iy)) / M1 * dzdy;
+          const double u1 = (1.0 * kPi * ix) / L1 * dzdx;
+          double gxv = 1.0, gyv = 1.0;
+          if (!(ix == 0 && iy == 0)) {
+            const double rr = u1 * u1 + v1 * v1;
+            const double upcc = std::exp(-std::sqrt(rr)) * (1.0 / std::sqrt(rr));
+            gxv = rxy * u1 * upcc;
+            gyv = ryx * v1 * upcc;
+          }
+          c->gx[(size_t)iy * H + ix] = gxv;
+          c->gy[(size_t)iy * H + ix] = gyv;
+        }
+    }
     if (c->up_tiled) {
       // pitches are whole 128-byte lines and avoid multiples of 1 KiB (HBM channel spread)
       auto pitch = [](int n, int per_line) {
@@ -3080,6 +3219,7 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
     if (hipMemcpy(c->d_up, up.data(), up.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(TCSEM_EDEVICE, "operator upload"));
   }
+  if (c->up_dense && (rc = build_dense(c))) return bail(rc);
   if ((rc = alloc_slots(c, 1))) return bail(rc);
   c->nbatch = 1;
   c->up64 = upcont_args<double>(c);
@@ -3120,6 +3260,7 @@ void tcsem_destroy(tcsem_ctx *c) {
   (void)hipFree(c->d_maps);
   (void)hipFree(c->d_up);
   (void)hipFree(c->d_work);
+  (void)hipFree(c->d_dn);
   (void)hipFree(c->d_scratch);
   (void)hipFree(c->d_rx);
   (void)hipFree(c->d_rxi);
@@ -3668,6 +3809,11 @@ hipError_t upcont_on_planes(tcsem_ctx *c, void *scr, const void *bz0, void *bxai
   u.G = w + 2 * c->sA;
   u.tbx = w + 2 * (c->sA + c->sG);
   u.tby = u.tbx + c->sX;
+  if (u.d.on) {  // at most kUpcontScratchBytes (choose_air)
+    u.d.P = (double *)scr;
+    u.d.Rx = u.d.P + u.d.sP;
+    u.d.Ry = u.d.P + 2 * u.d.sP;
+  }
   hipError_t e = launch_upcont<T>(u, 1, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   return e;

@@ -155,6 +155,48 @@ struct FftPlan {
   const double *bhat;    // m complex FFT of the conjugate chirp, scaled by 1/m (Bluestein only)
 };
 
+// The air boundary as matrix products (tcsem_upmat.hip): tables and work planes, all FP64 but for
+// the row operators kop (FP32 with kf32).
+struct DenseOp {
+  int on, kf32;              // on: 0 not built, 1 where it pays (dense_pays), 2 always
+  float kb, w, bm;           // MB of row operators, mega point passes of the tiled chain, MB of a march's step
+  int ldax, ldb, MP;         // pitches: ax (columns q = 2 kx + re/im), bx and by (columns i), P and R (rows j)
+  const double *ax;          // L (zero rows to a multiple of 16) x ldax
+  const double *bx, *by;     // 2 H (zero rows to a multiple of 4) x ldb
+  const void *kop;           // per kx: even block (ne x (ne + nyo)), odd block (no x (no + nye)), kstride entries
+  long long kstride;
+  const double *nt, *ns, *ng;  // y-Nyquist bin of By (null: odd M1)
+  double *P, *Rx, *Ry;       // per slot 2 H x MP, slot stride sP
+  long long sP;
+};
+// Whether the matrix form is faster than the tiled chain for a step of nslot slots.  It reads kb once per
+// step; the chain's time goes with its transforms' point passes w, but while the march takes longer
+// than the chain (bm: the march's bytes) the chain hides beside it and the operators' bytes do not.  The
+// line between was fitted to whole runs, us per step chain / matrix form (kb, w, bm for one slot):
+//   FP32 100 x 100 x 60 under 356 x 356 (7, 15, 25) 87 / 57; 320 x 320 x 60 under 576 x 576 (119, 65, 252)
+//     149 / 126; 320 x 320 x 160 (119, 65, 672) 224 / 245; 420 x 400 x 60 under 676 x 656 (217, 78, 413) 183 / 216;
+//     256 x 256 x 60 under 512 x 512 (68, 6, 161) 93 / 94; 200 x 200 x 160 under 712 x 712 (57, 65, 262) 167 / 131;
+//     300 x 300 x 60 under 556 x 556, 2 slots 217 / 192, 8 slots 761 / 544;
+//   FP64 100 x 100 x 60 103 / 68; 320 x 320 x 60 (238, 65, 504) 252 / 227; 420 x 400 x 60 (435, 78, 827) 342 / 362;
+//     360 x 350 x 160 under 616 x 606 (304, 70, 1653) 512 / 534; 300 x 300 x 60, 2 slots 402 / 325, 8 slots 1749 / 837.
+inline bool dense_line(bool fp32, float kb, float w, float bm) {
+  return fp32 ? 4.75f * w - 0.46f * bm + 30.f > kb : 6.75f * w - 0.175f * bm + 30.f > kb;
+}
+inline bool dense_pays(const DenseOp &d, bool fp32, int nslot) {
+  return d.on == 2 || (d.on == 1 && dense_line(fp32, d.kb, d.w * nslot, d.bm * nslot));
+}
+// Building them: the tables above, cosine/sine tables per ky (pitch ldy) and the folded gains.
+struct DenseBuild {
+  const double2 *tx, *ty;    // exp(2 pi i n / L1), n < L1; exp(pi i n / M1), n < 2 M1
+  double *ax, *bx, *by, *nt, *ns, *ng;
+  int ldax, ldb, ldy, Hy;
+  double *cw, *sw, *cs, *ss, *ce, *se;  // Hy x ldy
+  double *gx, *gy;           // H x Hy
+  void *kop;
+  long long kstride;
+  double dzdx, dzdy, rxy, ryx;
+};
+
 template <typename T>
 struct UpcontArgs {
   const T *bz0;            // plane origin (slot 0), row pitch pz
@@ -193,6 +235,7 @@ struct UpcontArgs {
   const int *xBx2N, *yo2N, *xo2N, *yBy2N;
   const int *yrows;        // the nyr regular rows (ascending) that the bilinear step reads
   int nyr;
+  DenseOp d;               // the matrix form (d.on), instead of either chain where it pays
 };
 
 // A launch whose dispatch packet records e0 at its start and e1 at its end when either is given;
@@ -243,6 +286,12 @@ hipError_t launch_gather(const GatherArgs &g, int is_b, int nslot, const MarchAr
 template <typename T>
 hipError_t launch_upcont(const UpcontArgs<T> &u, int nslot, hipStream_t s, hipEvent_t e0 = nullptr,
                          hipEvent_t e1 = nullptr, const UpcontArgs<T> *geo = nullptr, bool alone = false);
+// The same boundary in matrix form (u.d.on; three launches), and building its operators (u: the FP64 record
+// of the model's tables).
+template <typename T>
+hipError_t launch_dense(const UpcontArgs<T> &u, int nslot, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
+                        const UpcontArgs<T> *geo);
+hipError_t launch_dense_build(const DenseBuild &b, const UpcontArgs<double> &u, bool kf32, hipStream_t s);
 hipError_t launch_fill_zero(void *p, size_t bytes, hipStream_t s);
 // Work planes of the allocation-free upward continuation: a file-scope device array of
 // kUpcontScratchBytes per device (tcsem_upcont.hip).  upcont_scratch_init looks its address up on

@@ -782,6 +782,8 @@ hipError_t launch_lined(const UpcontArgs<T> &u, int nslot, hipStream_t s, hipEve
 template <typename T>
 hipError_t launch_upcont(const UpcontArgs<T> &u, int nslot, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
                          const UpcontArgs<T> *geo, bool alone) {
+  // a model batch's record says 2 or 0 (decided over its members)
+  if (dense_pays(u.d, sizeof(T) == 4, nslot)) return launch_dense<T>(u, nslot, s, e0, e1, geo);
   if (geo && !u.tiled) return hipErrorInvalidValue;  // model batches run the tiled chain only
   hipError_t e = geo ? launch_tiled<T, true>(u, nslot, s, e0, geo, alone)
                      : (u.tiled ? launch_tiled<T, false>(u, nslot, s, e0, nullptr, alone)
