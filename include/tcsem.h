@@ -245,10 +245,9 @@ int tcsem_sigma_table(const tcsem_ctx *ctx);
  * intermediate state stays on chip there), then the top levels of each step as usual.  The
  * results equal, bit for bit, those of one step at a time with an unchunked march (tested).
  * rows 0 turns it off.  Without a call the library decides at tcsem_begin: TCSEM_MARCH_PAIRS ("0"
- * or "rows,pf"), else the autotuner's choice for the batch size, else 12-row passes where they
- * give at least two workgroups per CU (14-row FP32 or 11-row FP64 passes where those leave fewer
- * idle CUs in the last round of workgroups); a call holds for the context's later runs.  Graph replays,
- * where on, take precedence.  Needs N >= 6.
+ * or "rows,pf"), else the autotuner's choice for the batch size, else, where 8-row passes give about
+ * half the CUs a workgroup, the height whose rounds of one workgroup per CU cost least (prefetch 2); a
+ * call holds for the context's later runs.  Graph replays, where on, take precedence.  Needs N >= 6.
  * tcsem_pair_info reports the setting and the pairs taken so far; tcsem_pair_timing the average
  * device time [ms] of the two-step pass alone (timing enabled; its top launches count in
  * tcsem_timing's t[0], per step). */
@@ -284,8 +283,8 @@ int tcsem_batch_enable_timing(tcsem_batch *batch, int on);
 int tcsem_batch_timing(tcsem_batch *batch, double t[3], long n[3]);
 /* Two steps per pass for the batch (no counterpart in the reference), as tcsem_set_pairs for a
  * context: rows 8, 10, 12, 14 or 16 (FP64: 8, 10, 11 or 12) at prefetch depth 1, or 0 (one step at a time), over
- * the library's choice (TCSEM_MARCH_PAIRS, the batch autotuner's pick, else 12-row passes when
- * the members' pass tiles give at least two workgroups per CU).  Pairs run when every member
+ * the library's choice (TCSEM_MARCH_PAIRS, the batch autotuner's pick, else as for a context over the
+ * members' pass tiles).  Pairs run when every member
  * still sampling is past its source wavelet and takes no sample after the pair's first step.
  * The results equal one step at a time, bit for bit (tested).  tcsem_batch_pair_info: the rows
  * of the last step call (0: one step at a time), the autotuner's pick (-1: not tuned) and the

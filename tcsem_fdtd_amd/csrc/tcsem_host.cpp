@@ -560,15 +560,53 @@ void apply_tiling(tcsem_ctx *c, int by, int pf, int nch) {
   c->sper = (c->stx * c->sty + 7) / 8;
 }
 
+int pass_tiles_x(int prec, int by, int L) {
+  const int w = pass_cols(prec / 8, by);
+  return (L + w - 1) / w;
+}
+int pass_tiles_y(int M, int by) { return (M + by - 5) / (by - 4); }
+
 // Tiles of the two-step pass (rows 0: pairs off).
 void pair_tiling(tcsem_ctx *c, int by, int pf) {
   const int L = c->g.info.L, M = c->g.info.M;
   c->pair_by = by;
   c->pair_pf = pf;
   if (!by) return;
-  c->pair_ntx = (L + kMarchLanes - 5) / (kMarchLanes - 4);
-  c->pair_nty = (M + by - 5) / (by - 4);
+  c->pair_ntx = pass_tiles_x(c->prec, by, L);
+  c->pair_nty = pass_tiles_y(M, by);
   c->pair_nper = (c->pair_ntx * c->pair_nty + 7) / 8;
+}
+
+// Default height of the two-step pass for a grid, a transmitter batch or a model batch (0: one step at a
+// time); tiles(b): its workgroups at b rows, state_mb: old and new state, MB, levels: of the deepest grid.
+// A compute unit holds one workgroup of a pass, so the pass takes rounds of `cu` of them, and a round the
+// time weighed here (us per level of 512 x 512 x 256, FP32 0.87 at 16 rows; fitted to 17 FP32 and 24 FP64 grids,
+// 90 x 90 to 512 x 512, 1 to 16 slots, where the pick is within 0.2% and 1% of the fastest height on average).
+// 10-row FP64 tiles weigh less alone in a round, where bandwidth is not what bounds them: 256 x 256 x 160, 10 / 11
+// rows 29.9 / 30.9 ms, against two rounds of 398 x 354 x 180, 88.5 / 86.7.  A state that stays in the 256 MB
+// memory-side cache makes the rows alone count (512 x 512 x 20, 200 steps, 8 to 16 rows: 27.6 to 28.3 ms).
+// Too few tiles leave the z-chunked march ahead, one step at a time / pass: FP32 140 x 140 x 120 (105 tiles of 8
+// rows) 15.5 / 16.6 ms, 160 x 160 x 100 (120) 12.3 / 12.5, 200 x 180 x 60 (180) 12.5 / 10.8, 256 x 256 x 160
+// (320) 20.7 / 19.6; FP64 120 x 120 x 160 (90) 15.4 / 18.6, 140 x 140 x 120 (105) 23.4 / 21.0, 256 x 256 x
+// 160 43.3 / 30.0.
+template <typename F>
+int pass_rows(int prec, F &&tiles, double state_mb, int cu) {
+  if (2 * tiles(8) < (prec == 32 ? 256 : 200) * (long long)cu / 256) return 0;
+  int best = 0;
+  double cost = 1e300;
+  for (int b : {8, 10, 11, 12, 14, 16}) {
+    if (!pair_rows_supported(prec, b)) continue;
+    const long long rounds = (tiles(b) + cu - 1) / cu;
+    double w = b;
+    if (state_mb > 256.0)
+      w = prec == 32 ? (b == 8 ? 12.8 : b == 10 ? 15.3 : b == 12 ? 16.5 : b == 14 ? 20.7 : 19.0)
+                     : (b == 8 ? 14.3 : b == 10 ? (rounds == 1 ? 15.4 : 16.2) : b == 11 ? 15.7 : 17.0);
+    if (rounds * w < cost) {
+      cost = rounds * w;
+      best = b;
+    }
+  }
+  return best;
 }
 
 // Tiling of an nbatch-transmitter step: the autotuned one for this batch size when there is
@@ -621,21 +659,12 @@ void choose_tiling(tcsem_ctx *c, int nbatch) {
   }
   apply_tiling(c, by, pf, nch);
   // Two steps per pass: tcsem_set_pairs' choice, else TCSEM_MARCH_PAIRS ("0", or "rows,pf"), else
-  // the autotuner's for this batch size, else 12-row passes at prefetch 1 when they give at least
-  // two workgroups per CU (faster than one step at a time on every such workload measured; fewer
-  // leave CUs idle, and the one-step march's z-chunks serve those grids better). The pass holds
-  // one workgroup per CU and a round of them takes about as long as the tile has rows, so 14-row
-  // (FP32) or 11-row (FP64) passes replace the 12-row ones where their rounds x rows is 5% or
-  // more smaller: a plane whose 12-row tiles leave the last round mostly empty (512 x 512).
-  int pby = 0, ppf = 1;
-  auto ptiles = [&](int b) {
-    return (long long)((L + kMarchLanes - 5) / (kMarchLanes - 4)) * ((M + b - 5) / (b - 4)) * nbatch;
-  };
-  if (ptiles(12) >= 2LL * cu) {
-    const int alt = c->prec == 32 ? 14 : 11;
-    auto cost = [&](int b) { return (double)((ptiles(b) + cu - 1) / cu) * b; };
-    pby = cost(alt) <= 0.95 * cost(12) ? alt : 12;
-  }
+  // the autotuner's for this batch size, else pass_rows' height at prefetch 2 (against 1: 256 x 256 x 160 FP32
+  // 119.3 / 120.7 ms, FP64 92.6 / 93.1, 512 x 512 x 256 177.0 / 177.3).
+  int ppf = 2;
+  int pby = pass_rows(
+      c->prec, [&](int b) { return (long long)pass_tiles_x(c->prec, b, L) * pass_tiles_y(M, b) * nbatch; },
+      10.0 * L * M * N * nbatch * c->esz * 1e-6, cu);
   if (c->tune_nbatch == nbatch) {
     pby = c->tune_pair_by;
     ppf = c->tune_pair_pf;
@@ -2049,9 +2078,6 @@ int batch_work_list(tcsem_batch *b, const std::vector<int> &tiles, int2 **d, siz
   return TCSEM_OK;
 }
 
-int pass_tiles_x(int L) { return (L + kMarchLanes - 5) / (kMarchLanes - 4); }
-int pass_tiles_y(int M, int by) { return (M + by - 5) / (by - 4); }
-
 // pby > 0: also the records of two steps per pass with pby-row tiles (each member's intermediate
 // state allocated on first use).
 template <typename T>
@@ -2145,7 +2171,7 @@ int batch_records(tcsem_batch *b, int by, int pf, MarchArgs<T> &la, UpcontArgs<T
       const long long org = c->PX + c->xm, fs = c->fstride * c->nslots, ps = c->pstride * c->nslots;
       T *fm = (T *)c->d_mid, *pl = (T *)c->d_planes;
       const tcsem_grid_info &I = c->g.info;
-      tiles[q] = pass_tiles_x(I.L) * pass_tiles_y(I.M, pby);
+      tiles[q] = pass_tiles_x(b->prec, pby, I.L) * pass_tiles_y(I.M, pby);
       for (int p = 0; p < 2; ++p) {
         const MarchArgs<T> &r = rec[(size_t)p * nm + q];
         PairArgs<T> pr{};
@@ -2158,7 +2184,7 @@ int batch_records(tcsem_batch *b, int by, int pf, MarchArgs<T> &la, UpcontArgs<T
         pr.cs2 = pl + 5 * ps + org;
         pr.cc2 = pl + 6 * ps + org;
         pr.rows = pby;
-        pr.ntx = pass_tiles_x(I.L);
+        pr.ntx = pass_tiles_x(b->prec, pby, I.L);
         pr.nty = pass_tiles_y(I.M, pby);
         prec[(size_t)p * nm + q] = pr;
         MarchArgs<T> ta = r;  // step A's top launch and surface: old state -> intermediate state
@@ -2377,12 +2403,20 @@ int batch_pair_rows(tcsem_batch *b) {
     if (std::sscanf(e, "%d,%d", &r, &q) >= 1 && (r == 0 || (pair_rows_supported(b->prec, r) && q == 1))) return r;
   }
   if (b->pair_tuned >= 0) return b->pair_tuned;
-  const int rows = b->prec == 64 ? 8 : 12;
-  long long tiles = 0;
+  auto tiles = [&](int rows) {
+    long long n = 0;
+    for (size_t q = 0; q < b->m.size(); ++q)
+      if (b->active[q])
+        n += (long long)pass_tiles_x(b->prec, rows, b->m[q]->g.info.L) * pass_tiles_y(b->m[q]->g.info.M, rows);
+    return n;
+  };
+  double mb = 0.0;
   for (size_t q = 0; q < b->m.size(); ++q)
-    if (b->active[q])
-      tiles += (long long)pass_tiles_x(b->m[q]->g.info.L) * pass_tiles_y(b->m[q]->g.info.M, rows);
-  return tiles >= 2LL * device_cus() ? rows : 0;
+    if (b->active[q]) {
+      const tcsem_grid_info &I = b->m[q]->g.info;
+      mb += 10.0 * I.L * I.M * I.N * (b->prec / 8) * 1e-6;
+    }
+  return pass_rows(b->prec, tiles, mb, device_cus());
 }
 
 // Orders the batch's work before what is issued next on the batch's and the members' streams.

@@ -30,6 +30,19 @@ constexpr int kSurfaceOwnX = kMarchLanes - 2;
 constexpr int kSurfaceRows = 8;
 constexpr int kMaxChunks = 16;  // z-chunks of one lower march launch
 
+// Columns that a workgroup of the two-step pass owns of its 64 lanes (two or more halo columns each side;
+// esz: bytes of an element).  At 48 FP32 or 56 FP64 columns a row of the tile is whole 64-byte segments, which
+// no other workgroup writes a part of; at 56 or 60 FP32 columns neighbours share segments, which cost
+// bandwidth unless their stores merge in L2.  Pass of 512 x 512 x 256 FP32, us per launch: 16 rows of 60
+// columns 934 non-temporal, 836 cached; 14 rows 873, 751; 16 rows of 48 columns 713, 729.  Sixteen slots of
+// 256 x 256 x 160, 240 steps, ms: 12 rows of 60 318, 291, of 56 cached 287, 16 rows of 48 301.  Where all
+// tiles run at once (8 and 10 rows are for those grids) the lanes count for more: 256 x 256 x 160, 1000 steps,
+// 10 rows of 60 120.7, cached 123.5, of 48 (two rounds) 177.6.  FP64 398 x 354 x 180, 300 steps: 11 rows of 60
+// 134.0, of 56 128.7, six uneven models 128.8, 113.3.
+constexpr int pass_cols(int esz, int rows) {
+  return esz == 8 || rows == 12 ? 56 : rows == 16 ? 48 : 60;
+}
+
 // One injected E cell: E[comp](k, j, i) -= amp * w each source step (ElectricalFiled.cu:347-475).
 // The same record lists the B cells a source step recomputes (comp 3 Bx, 4 By; w unused).
 struct SrcCell {

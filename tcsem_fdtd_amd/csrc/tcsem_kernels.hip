@@ -27,14 +27,17 @@
 
 namespace tcsem {
 
-// Running Bz integral: plain FP64, or compensated (TwoSum) FP32.
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// Running Bz integral, s + a b: plain FP64, or compensated (TwoSum of the unrounded product) FP32.
 template <typename T>
 struct Acc;
 template <>
 struct Acc<double> {
   double s;
   __device__ void init() { s = 0.0; }
-  __device__ void add(double x) { s += x; }
+  __device__ void add(double a, double b) { s = fma_(a, b, s); }
   __device__ double val() const { return s; }
   __device__ void save(double *ps, double *, unsigned off) const { *(double *)((char *)ps + off) = s; }
   __device__ void load(const double *ps, const double *, unsigned off) { s = *(const double *)((const char *)ps + off); }
@@ -51,53 +54,54 @@ struct Acc<float> {
     s = *(const float *)((const char *)ps + off);
     c = *(const float *)((const char *)pc + off);
   }
-  __device__ void add(float x) {
-    const float t = s + x;
+  __device__ void add(float a, float b) {
+    const float t = fma_(a, b, s);
     const float bp = t - s;
-    c += (s - (t - bp)) + (x - bp);
+    c += (s - (t - bp)) + fma_(a, b, -bp);
     s = t;
   }
   __device__ float val() const { return s + c; }
 };
 
+// Every update is spelled out in fused and plain operations, so that the one-step march, the two-step pass and
+// the surface and source kernels round alike.
+// a ra - b rb and a ra + b rb
+template <typename T>
+__device__ __forceinline__ T curl2(T a, T ra, T b, T rb) {
+  return fma_(a, ra, -(b * rb));
+}
+template <typename T>
+__device__ __forceinline__ T div2(T a, T ra, T b, T rb) {
+  return fma_(a, ra, b * rb);
+}
+
 // DuFort-Frankel update E <- (2l - s dt)/(2l + s dt) E + 4 dt/(2l + s dt) curl / mu0
 // (ElectricalFiled.cu:138-139), written with x = s dt / (2l): E <- (1-x)/(1+x) E + c4/(1+x) curl,
-// c4 = 4 dt / (2l mu0).  FP64 fields: one FP64 division per update.  FP32 fields: the reciprocal
-// of 1+x from v_rcp_f32 refined by one Newton step (error below one ulp, unbiased in sign).
-struct Coef64 {
-  double q2, c4;  // dt/(2l), 4 dt/(2l mu0)
+// c4 = 4 dt / (2l mu0).  s4 is the plain sum of the four cells that the conductivity is averaged over (q2 carries
+// the quarter).
+// FP32: the reciprocal of 1+x from v_rcp_f32 refined by one Newton step (error below one ulp, unbiased in sign).
+// Its operations stay as they are: forms with one or two fewer moved the traces of receivers far below the
+// source by up to 1e-4, the round-off of the strong field near the source.
+// FP64: ((1-x) E + c4 curl) / (1+x) by the hardware reciprocal, a Newton step and the remainder of the quotient:
+// within an ulp, after two roundings where separate factors took three; 16 issue slots against 24 with an
+// IEEE division of 1 by 1+x (pass of 398 x 354 x 180 and its like: see pass_cols).
+template <typename T>
+struct Coef {
+  T q2, c4;  // dt/(8l), 4 dt/(2l mu0)
 };
-__device__ inline double df_new(double e, double sig, const Coef64 &k, double curl) {
-  const double x = sig * k.q2;
-  const double r = 1.0 / (1.0 + x);
-  return (1.0 - x) * r * e + k.c4 * r * curl;
+__device__ __forceinline__ float df_new(float e, float s4, const Coef<float> &k, float curl) {
+  const float d = fma_(s4, k.q2, 1.0f), m = fma_(-s4, k.q2, 1.0f);
+  const float r0 = __builtin_amdgcn_rcpf(d), r = r0 * fma_(-d, r0, 2.0f);
+  return fma_(m * r, e, (k.c4 * r) * curl);
 }
-struct Coef32 {
-  float q2, c4;
-};
-__device__ inline float df_new(float e, float sig, const Coef32 &k, float curl) {
-  const float x = sig * k.q2;
-  const float d = 1.0f + x;
-  float r = __builtin_amdgcn_rcpf(d);
-  r = r * (2.0f - d * r);
-  return (1.0f - x) * r * e + k.c4 * r * curl;
+__device__ __forceinline__ double df_new(double e, double s4, const Coef<double> &k, double curl) {
+  const double d = fma_(s4, k.q2, 1.0), t = fma_(fma_(-s4, k.q2, 1.0), e, k.c4 * curl);
+  const double r0 = __builtin_amdgcn_rcp(d), r = fma_(r0, fma_(-d, r0, 1.0), r0), q = t * r;
+  return fma_(fma_(-d, q, t), r, q);
 }
 template <typename T>
-struct CoefOf;
-template <>
-struct CoefOf<double> {
-  using type = Coef64;
-};
-template <>
-struct CoefOf<float> {
-  using type = Coef32;
-};
-template <typename T>
-__device__ inline typename CoefOf<T>::type make_coef(double lam, double dt) {
-  typename CoefOf<T>::type k;
-  k.q2 = (T)(dt / (2.0 * lam));
-  k.c4 = (T)(4.0 * dt / (2.0 * lam * kMu0));
-  return k;
+__device__ inline Coef<T> make_coef(double lam, double dt) {
+  return {(T)(dt / (8.0 * lam)), (T)(4.0 * dt / (2.0 * lam * kMu0))};
 }
 
 template <typename T>
@@ -187,6 +191,41 @@ __device__ __forceinline__ double bld(__amdgpu_buffer_rsrc_t r, unsigned off, do
   typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
   const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, AUX);
   return __longlong_as_double((long long)(((unsigned long long)w.y << 32) | w.x));
+}
+
+// The same with the level in the scalar offset, which the range check leaves out: a lane's offset of kDrop
+// still drops the access.
+template <int AUX>
+__device__ __forceinline__ float bld(__amdgpu_buffer_rsrc_t r, unsigned off, float, int so) {
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)off, so, AUX));
+}
+template <int AUX>
+__device__ __forceinline__ double bld(__amdgpu_buffer_rsrc_t r, unsigned off, double, int so) {
+  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, so, AUX);
+  return __longlong_as_double((long long)(((unsigned long long)w.y << 32) | w.x));
+}
+template <int AUX>
+__device__ __forceinline__ void bsto_at(__amdgpu_buffer_rsrc_t r, unsigned off, int so, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)off, so, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void bsto_at(__amdgpu_buffer_rsrc_t r, unsigned off, int so, double v) {
+  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  u32x2 w;
+  w.x = (unsigned)b;
+  w.y = (unsigned)(b >> 32);
+  __builtin_amdgcn_raw_buffer_store_b64(w, r, (int)off, so, AUX);
+}
+
+// f(0), f(1) .. f(n-1) with compile-time indices
+template <int n, typename F>
+__device__ __forceinline__ void unrolled(F &&f) {
+  if constexpr (n > 0) {
+    unrolled<n - 1>(f);
+    f(std::integral_constant<int, n - 1>{});
+  }
 }
 
 // Per-lane geometry shared by the march and the surface kernel.  Every lane computes every
@@ -340,6 +379,7 @@ k_march(const MarchArgs<T> la, const MarchArgs<T> *geo) {
   const int hsl = lx == 0 ? 0 : (lx == kMarchLanes - 1 ? LW - 1 : sl);
   const bool left = lx == 0, right = lx == kMarchLanes - 1;
   const int lym = max(ly - 1, 0), lyp = min(ly + 1, BY - 1);
+  const auto cf = make_coef<T>(a.lam, a.dt);
   const T rdx = a.rdx[ic + 1], rdx2 = a.rdx2[ic + 1], rdy = a.rdy[jc + 1], rdy2 = a.rdy2[jc + 1];
   const T rdxL = a.rdx[max(i0 - 1, -1) + 1], rdx2R = a.rdx2[min(iR, L + 1) + 1];
   // slots in grid y: each slot's tiles run as XCD-contiguous bands one slot after another, which
@@ -373,7 +413,6 @@ k_march(const MarchArgs<T> la, const MarchArgs<T> *geo) {
   const __amdgpu_buffer_rsrc_t rezi = rsrc_of((void *)ezi, fbytes);
   const bool ezrow = ly >= 1;
   const bool erow = ly >= 1 && ly <= BY - 2;
-  const auto cf = make_coef<T>(a.lam, a.dt);
   const T dtb = (T)a.dtb, zero = 0;
 
   // A ring of PF+2 register slots holds level k (cur), level k-1 (nxt) and the PF-1 levels below
@@ -498,8 +537,8 @@ k_march(const MarchArgs<T> la, const MarchArgs<T> *geo) {
     const T bx_k = cur.bx, by_k = cur.by, bx_m = nxt.bx, by_m = nxt.by;
     // (a) Bz_old(k) = Bz_old(k+1) + dz(k) div_h(B_old(k)), for the lane's column and column i0-1
     // (the opening level of an upper chunk starts from Bz_old(k) itself: its increment is zero)
-    bz.add(dzk * ((sBx[p][ly][slp] - bx_k) * rdx + (sBy[p][lyp][sl] - by_k) * rdy));
-    bzL.add(dzk * ((bx_k - cur.hbx) * rdxL + (sBy[p][lyp][0] - cur.hby) * rdy));
+    bz.add(dzk, div2(sBx[p][ly][slp] - bx_k, rdx, sBy[p][lyp][sl] - by_k, rdy));
+    bzL.add(dzk, div2(bx_k - cur.hbx, rdxL, sBy[p][lyp][0] - cur.hby, rdy));
     const T bzk = bz.val();
     sBz[ly][sl] = bzk;
     sBz[ly][left ? 0 : sl] = left ? bzL.val() : bzk;
@@ -513,14 +552,14 @@ k_march(const MarchArgs<T> la, const MarchArgs<T> *geo) {
     // (c) Ez(k) on the tile rows and the +y halo row; lane 63 also for column i0+64
     T ezn, ezr;
     {
-      const T s4 = (T)0.25 * (sS[p][lym][slm] + sS[p][lym][sl] + sS[p][ly][slm] + sS[p][ly][sl]);
-      const T curl = (by_k - sBy[p][ly][slm]) * rdx2 - (bx_k - sBx[p][lym][sl]) * rdy2;
-      ezn = vEzAny ? df_new(ezo, s4, cf, curl) : zero;
+      const T s4 = sS[p][lym][slm] + sS[p][lym][sl] + sS[p][ly][slm] + sS[p][ly][sl];
+      const T v = df_new(ezo, s4, cf, curl2(by_k - sBy[p][ly][slm], rdx2, bx_k - sBx[p][lym][sl], rdy2));
+      ezn = vEzAny ? v : zero;
     }
     {
-      const T s4 = (T)0.25 * (sS[p][lym][LW - 2] + sS[p][lym][LW - 1] + sS[p][ly][LW - 2] + sS[p][ly][LW - 1]);
-      const T curl = (cur.hby - by_k) * rdx2R - (cur.hbx - sBx[p][lym][LW - 1]) * rdy2;
-      ezr = vEzR ? df_new(cur.hez, s4, cf, curl) : zero;
+      const T s4 = sS[p][lym][LW - 2] + sS[p][lym][LW - 1] + sS[p][ly][LW - 2] + sS[p][ly][LW - 1];
+      const T v = df_new(cur.hez, s4, cf, curl2(cur.hby - by_k, rdx2R, cur.hbx - sBx[p][lym][LW - 1], rdy2));
+      ezr = vEzR ? v : zero;
     }
     sEz[ly][sl] = ezn;
     sEz[ly][right ? LW - 1 : sl] = right ? ezr : ezn;
@@ -528,23 +567,21 @@ k_march(const MarchArgs<T> la, const MarchArgs<T> *geo) {
     // (d) Ex(k), Ey(k)
     T exn, eyn;
     {
-      const T sxk = (T)0.5 * (sS[p][lym][sl] + sS[p][ly][sl]);
-      const T sxm = (T)0.5 * (sS[q][lym][sl] + sS[q][ly][sl]);
-      const T ave = (T)0.5 * (sxk + sxm);
-      const T curl = (bzk - sBz[lym][sl]) * rdy2 - (by_k - by_m) * rdz2k;
-      exn = vEx ? df_new(exo, ave, cf, curl) : zero;
+      const T s4 = (sS[p][lym][sl] + sS[p][ly][sl]) + (sS[q][lym][sl] + sS[q][ly][sl]);
+      const T v = df_new(exo, s4, cf, curl2(bzk - sBz[lym][sl], rdy2, by_k - by_m, rdz2k));
+      exn = vEx ? v : zero;
     }
     {
-      const T s4 = (T)0.25 * (sS[p][ly][slm] + sS[p][ly][sl] + sS[q][ly][slm] + sS[q][ly][sl]);
-      const T curl = (bx_k - bx_m) * rdz2k - (bzk - sBz[ly][slm]) * rdx2;
-      eyn = vEy ? df_new(eyo, s4, cf, curl) : zero;
+      const T s4 = sS[p][ly][slm] + sS[p][ly][sl] + sS[q][ly][slm] + sS[q][ly][sl];
+      const T v = df_new(eyo, s4, cf, curl2(bx_k - bx_m, rdz2k, bzk - sBz[ly][slm], rdx2));
+      eyn = vEy ? v : zero;
     }
     bsto(rex, off, vEx && st, exn);
     bsto(rey, off, vEy && st, eyn);
     __syncthreads();
     // (e) Bx(k), By(k) from E_new(k), E_new(k+1)
-    const T bxn = bx_k + dtb * ((ey_n1 - eyn) * rdzk - (sEz[lyp][sl] - ezn) * rdy);
-    const T byn = by_k + dtb * ((sEz[ly][slp] - ezn) * rdx - (ex_n1 - exn) * rdzk);
+    const T bxn = fma_(dtb, curl2(ey_n1 - eyn, rdzk, sEz[lyp][sl] - ezn, rdy), bx_k);
+    const T byn = fma_(dtb, curl2(sEz[ly][slp] - ezn, rdx, ex_n1 - exn, rdzk), by_k);
     bsto(rbx, off, vBx && st, bxn);
     bsto(rby, off, vBy && st, byn);
     if constexpr (IB) {  // dzk is zero on a level the launch does not store
@@ -574,7 +611,7 @@ k_march(const MarchArgs<T> la, const MarchArgs<T> *geo) {
     return;
   }
   // Bz_old(0) for the upward continuation and the surface level (level 0 sits in buffer 0)
-  bz.add(sZ[0] * ((sBx[0][ly][slp] - bx_last) * rdx + (sBy[0][lyp][sl] - by_last) * rdy));
+  bz.add(sZ[0], div2(sBx[0][ly][slp] - bx_last, rdx, sBy[0][lyp][sl] - by_last, rdy));
   if (own) sto(a.bz0 + po, colb, bz.val());
 }
 
@@ -587,22 +624,27 @@ k_march(const MarchArgs<T> la, const MarchArgs<T> *geo) {
 // (read sigma and the old state once, write the new state once per two steps), for a halo ring
 // two cells wide instead of one.
 // Every quantity is the one-step march's expression in the same operation order, so the two
-// steps give the bits of two one-step passes.  The tile is 64 lanes (columns i0-2 .. i0+61) by
-// BY rows (j0-2 .. j0+BY-3): step A is exact on lanes and rows 1 .. 62 / BY-2 (the neighbours its
-// curls read are one cell further out), step B on lanes 2 .. 61 and rows 2 .. BY-3, the cells a
-// workgroup owns.  Cells outside the grid read and compute as zero, as memory holds them.
+// steps give the bits of two one-step passes.  The tile is 64 lanes by BY rows (j0-2 .. j0+BY-3), of which a
+// workgroup owns pass_cols columns in the middle and BY - 4 rows: step A is exact one ring further out than
+// step B (the neighbours its curls read are one cell further out still).  Cells outside the grid compute as zero,
+// as memory holds them.
+// Bound by HBM where its tiles come in several rounds (512 x 512 x 256 FP32: 3.1 GB in 0.72 ms) and by the chain
+// of a level's phases where they come in one.  147 vector instructions per lane and level (FP32), against 210
+// with selects for the grid's edge, address arithmetic per access and the two-level delay lines moved
+// between registers: same FP32 time at the old 60-column tiles, whose shared store segments bound it, but what let
+// 48 and 56 columns pay, and 1.3 to 1.5 times faster FP64 passes (with the cheaper division).
 // Per iteration, three phases with a barrier after the first two (the third runs into the next
 // iteration's first, which touches none of its LDS):
 //   P1  A: Bz sum of level k (B_old of level k: y-neighbours from LDS); stage B_old and sigma of
 //          level k-1; loads of level k-1-PF.   B: Bz sum of level k+2 (intermediate B).
 //   P2  A: intermediate E of level k.   B: new E of level k+2 (stored).
 //   P3  A: intermediate B of level k (into LDS for step B).   B: new B of level k+2 (stored).
-// Step B idles on the first two iterations (levels N+1, N: dz 0, nothing stored, inputs zero)
-// and step A on the last (k = 1: nothing kept), so every iteration runs the same code.  The
+// Step B idles on the first two iterations (levels N+1, N: zero inputs, zeros stored into level N-1 before its
+// own values) and step A on the last (k = 1: nothing kept), so every iteration runs the same code.  The
 // lower pass never reads level 0 of the old state (the previous pair's surface kernel writes it).
 // The same register of the lane to the left (l-1) or right (l+1) in the wavefront, by a DPP
 // whole-wave shift (wave_shr:1, wave_shl:1); the lanes past either end read 0.  The pass's rows
-// are single wavefronts, so its x-neighbours need no LDS round trip (in FP32, half its LDS reads).
+// are single wavefronts, so its x-neighbours need no LDS round trip (half its LDS reads).
 constexpr int kDppWaveShl1 = 0x130, kDppWaveShr1 = 0x138;
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
@@ -654,7 +696,9 @@ __global__ void __launch_bounds__(kMarchLanes *BY) k_march2(const PairArgs<T> la
     if (tile >= pa.ntx * pa.nty) return;
   }
   const MarchArgs<T> &a = pa.a;
-  constexpr int W = kMarchLanes, TX = W - 4, TY = BY - 4;
+  constexpr int W = kMarchLanes, TX = pass_cols((int)sizeof(T), BY), TY = BY - 4, X0 = (W - TX) / 2;
+  // partial 64-byte segments are left to merge in L2 (pass_cols)
+  constexpr int kSt = TX * sizeof(T) % 64 == 0 || BY <= 10 ? kNT : 0;
   extern __shared__ __align__(16) unsigned char zdyn[];  // 3 N entries of T
   __shared__ T sBx[2][BY][W], sBy[2][BY][W], sS[2][BY][W];
   __shared__ T sB1x[2][BY][W], sB1y[2][BY][W];
@@ -664,51 +708,48 @@ __global__ void __launch_bounds__(kMarchLanes *BY) k_march2(const PairArgs<T> la
   const int lx = threadIdx.x;
   const int ly = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // one wave per row
   const int L = a.L, M = a.M, N = a.N;
-  const int i = tx * TX - 2 + lx, j = ty * TY - 2 + ly;
+  const int i = tx * TX - X0 + lx, j = ty * TY - 2 + ly;
   // grid cells of each component (zero outside, as memory holds them): Ex i in [0,L) j in [1,M),
   // Ey and Bx i in [1,L) j in [0,M), Ez i in [1,L) j in [1,M), By as Ex
   const bool xin = i >= 0 && i < L, xin1 = i >= 1 && i < L, yin = j >= 0 && j < M, yin1 = j >= 1 && j < M;
-  const bool dEx = xin && yin1, dEy = xin1 && yin, dEz = xin1 && yin1, dBx = dEy, dBy = dEx;
-  const bool own = lx >= 2 && lx < W - 2 && ly >= 2 && ly < BY - 2;
+  const bool dEx = xin && yin1, dEy = xin1 && yin, dEz = xin1 && yin1;
+  const bool own = lx >= X0 && lx < X0 + TX && ly >= 2 && ly < BY - 2;
   const int ic = min(max(i, -1), L + 1), jc = min(max(j, -1), M + 1);
   const unsigned colb = (unsigned)((jc + 1) * a.PX + a.xm + ic) * (unsigned)sizeof(T);
-  const int lxm = max(lx - 1, 0), lxp = min(lx + 1, W - 1), lym = max(ly - 1, 0), lyp = min(ly + 1, BY - 1);
-  const T rdx = a.rdx[ic + 1], rdx2 = a.rdx2[ic + 1], rdy = a.rdy[jc + 1], rdy2 = a.rdy2[jc + 1];
+  const int lym = max(ly - 1, 0), lyp = min(ly + 1, BY - 1);
+  const auto cfA = make_coef<T>(a.lam, a.dt), cfB = make_coef<T>(pa.lamB, pa.dtB);
+  const T dtbA = (T)a.dtb, dtbB = (T)pa.dtbB, zero = 0;
+  const T rdx = a.rdx[ic + 1], rdy = a.rdy[jc + 1];
+  // Ez's curl coefficients are zero where it has no cell, so that with its old value dropped there too the
+  // update gives the zero its neighbours need without a select.  Ex and Ey off the grid are read by By and Bx
+  // off the grid only, which are set to zero.
+  const T rdx2 = a.rdx2[ic + 1], rdy2 = a.rdy2[jc + 1], zx = dEz ? rdx2 : zero, zy = dEz ? rdy2 : zero;
   const int slot = GEO ? 0 : (int)blockIdx.y;  // a model batch's records point at each member's slot 0
-  // x-neighbours by lane shifts (FP32), or from LDS (FP64: an x-neighbour from a lane shift lets
-  // the compiler fuse the other product of a curl into its FMA, which would round differently
-  // from the one-step march; the conductivity sums, which have no products, shift in both)
-  constexpr bool kX = sizeof(T) == 4;
   const long long fo = (long long)slot * a.fstride - (a.PX + a.xm);  // allocation base of the slot
   const long long po = (long long)slot * a.pstride - (a.PX + a.xm);
-  const T *__restrict__ bxi = a.bxi + fo;
-  const T *__restrict__ byi = a.byi + fo;
-  const T *__restrict__ sig = a.sig - (a.PX + a.xm);
-  const unsigned char *__restrict__ sig8 = S8 ? a.sig8 - (a.PX + a.xm) : nullptr;
+  constexpr unsigned kEsh = sizeof(T) == 8 ? 3 : 2;
   const unsigned PSb = (unsigned)a.PS * (unsigned)sizeof(T);
   const unsigned fbytes = (unsigned)(a.fstride * (long long)sizeof(T));
   const __amdgpu_buffer_rsrc_t rex = rsrc_of(a.ex + fo, fbytes), rey = rsrc_of(a.ey + fo, fbytes),
                                rez = rsrc_of(a.ez + fo, fbytes), rbx = rsrc_of(a.bx + fo, fbytes),
                                rby = rsrc_of(a.by + fo, fbytes);
-  const __amdgpu_buffer_rsrc_t mex = rsrc_of(pa.mex + fo, fbytes), mey = rsrc_of(pa.mey + fo, fbytes),
-                               mez = rsrc_of(pa.mez + fo, fbytes), mbx = rsrc_of(pa.mbx + fo, fbytes),
-                               mby = rsrc_of(pa.mby + fo, fbytes);
-  // old E: step A computes Ex, Ey on rows 1 .. BY-2 and Ez on rows 1 .. BY-1 (row 0 only sums Bz)
-  const __amdgpu_buffer_rsrc_t rexi = rsrc_of((void *)(a.exi + fo), fbytes),
-                               reyi = rsrc_of((void *)(a.eyi + fo), fbytes),
-                               rezi = rsrc_of((void *)(a.ezi + fo), fbytes);
+  // Loads and stores take the column in the lane's offset and the level in the scalar one, so that a level
+  // costs no address arithmetic; the resources of the old Ex, Ey drop whole rows (step A computes them on rows 1
+  // .. BY-2 and Ez on rows 1 .. BY-1; row 0 only sums Bz), the lanes' offsets the cells off the grid or not owned.
   const bool erow = ly >= 1 && ly <= BY - 2, ezrow = ly >= 1;
-  // the work each row's wave does (uniform branches): step A's Bz sum on rows 0 .. BY-2, its Ez on
-  // rows 1 .. BY-1, its Ex, Ey and B on rows 1 .. BY-2; step B's Bz sum on rows 1 .. BY-3, its Ez
-  // on rows 2 .. BY-2, its Ex, Ey and B (the stored cells) on rows 2 .. BY-3 -- what the owned
-  // cells read, one ring further out for step A
-  const bool rBzA = ly <= BY - 2, rA = ly >= 1 && ly <= BY - 2;
-  const bool rBzB = ly >= 1 && ly <= BY - 3, rEzB = ly >= 2 && ly <= BY - 2, rB = ly >= 2 && ly <= BY - 3;
-  const auto cfA = make_coef<T>(a.lam, a.dt);
-  const auto cfB = make_coef<T>(pa.lamB, pa.dtB);
-  const T dtbA = (T)a.dtb, dtbB = (T)pa.dtbB, zero = 0;
+  const __amdgpu_buffer_rsrc_t rbxi = rsrc_of((void *)(a.bxi + fo), fbytes), rbyi = rsrc_of((void *)(a.byi + fo), fbytes),
+                               rexi = rsrc_of((void *)(a.exi + fo), erow ? fbytes : 0u),
+                               reyi = rsrc_of((void *)(a.eyi + fo), erow ? fbytes : 0u),
+                               rezi = rsrc_of((void *)(a.ezi + fo), fbytes);
+  const __amdgpu_buffer_rsrc_t rsg =
+      S8 ? rsrc_of((void *)(a.sig8 - (a.PX + a.xm)), (unsigned)((long long)N * a.PS))
+         : rsrc_of((void *)(a.sig - (a.PX + a.xm)), (unsigned)((long long)N * a.PS * (long long)sizeof(T)));
+  const unsigned lEz = ezrow && dEz ? colb : kDrop;
+  const unsigned sEx = own && dEx ? colb : kDrop, sEy = own && dEy ? colb : kDrop, sEzo = own && dEz ? colb : kDrop;
+  // step B's E on rows 2 .. BY-2 (its own cells and the Ez above them); the other work is small against its
+  // branches and runs on every row, on values no owned cell reads
+  const bool rB = ly >= 2 && ly <= BY - 2;
   constexpr int S = PF + 2;
-  constexpr unsigned kEsh = sizeof(T) == 8 ? 3 : 2;
   constexpr int klo = 2, lfloor = 1;
   const int khi = N - 1;
   using LvT = Lv2<T, S8>;
@@ -718,187 +759,142 @@ __global__ void __launch_bounds__(kMarchLanes *BY) k_march2(const PairArgs<T> la
   T *sZ = (T *)zdyn;
   for (int q = ly * W + lx; q < 3 * N; q += W * BY) sZ[q] = a.dzt[q];
   auto load = [&](int lv) {
-    const unsigned o = (unsigned)max(lv, lfloor) * PSb + colb;
+    const int lc = max(lv, lfloor), o = lc * (int)PSb;
     LvT v;
-    v.bx = ldo(bxi, o);
-    v.by = ldo(byi, o);
+    v.bx = bld<0>(rbxi, colb, zero, o);
+    v.by = bld<0>(rbyi, colb, zero, o);
     if constexpr (S8)
-      v.s = ldo(sig8, o >> kEsh);
+      v.s = __builtin_amdgcn_raw_buffer_load_b8(rsg, (int)(colb >> kEsh), lc * (int)a.PS, 0);
     else
-      v.s = ldo(sig, o);
-    v.ex = bld<0>(rexi, erow ? o : kDrop, T(0));
-    v.ey = bld<0>(reyi, erow ? o : kDrop, T(0));
-    v.ez = bld<0>(rezi, ezrow ? o : kDrop, T(0));
+      v.s = bld<0>(rsg, colb, zero, o);
+    v.ex = bld<0>(rexi, colb, zero, o);
+    v.ey = bld<0>(reyi, colb, zero, o);
+    v.ez = bld<0>(rezi, lEz, zero, o);
     return v;
   };
   LvT R[S];
 #pragma unroll
   for (int d = 0; d < S - 1; ++d) R[d] = load(khi - d);
-  auto stage = [&](const int k, const LvT &v) -> T {  // B_old and sigma of level k into LDS
-    sBx[k & 1][ly][lx] = v.bx;
-    sBy[k & 1][ly][lx] = v.by;
+  auto stage = [&](const int p, const LvT &v) -> T {  // B_old and sigma of a level into LDS buffer p
+    sBx[p][ly][lx] = v.bx;
+    sBy[p][ly][lx] = v.by;
     T sv;
     if constexpr (S8)
       sv = sLut[v.s];
     else
       sv = v.s;
-    sS[k & 1][ly][lx] = sv;
-    return sv;  // the lane's own conductivity of level k
+    sS[p][ly][lx] = sv;
+    return sv;  // the lane's own conductivity
   };
   // step B's inputs of its idle iterations read as zero (each lane clears its own cells)
   sB1x[0][ly][lx] = sB1x[1][ly][lx] = zero;
   sB1y[0][ly][lx] = sB1y[1][ly][lx] = zero;
   __syncthreads();  // the table sLut
-  T sgk = stage(khi, R[0]);  // the lane's conductivity of level k
+  const T sg0 = stage(0, R[0]);
   Acc<T> bzA, bzB;  // running Bz sums of the old and of the intermediate B
   bzA.init();
   bzB.init();
-  // intermediate B of levels k+2 (c) and k+1 (n) and intermediate E of levels k+2 (c) and k+1 (n)
-  // of this lane's column; new E of level k+3 (step B's level below)
-  T b1xc = 0, b1yc = 0, b1xn = 0, b1yn = 0;
-  T e1xc = 0, e1yc = 0, e1zc = 0, e1xn = 0, e1yn = 0, e1zn = 0;
-  T e2x = 0, e2y = 0;
-  // conductivity averages (Ez, Ex, Ey) of levels k+2 (c) and k+1 (n)
-  T azc = 0, axc = 0, ayc = 0, azn = 0, axn = 0, ayn = 0;
+  // Of this lane's column, by iteration parity: intermediate B and E and the conductivity sums (Ez, Ex, Ey) of
+  // levels k+2 (this parity, replaced by level k's at the end) and k+1 (the other).  new E of level k+3.
+  T b1x[2] = {zero, zero}, b1y[2] = {zero, zero};
+  T e1x[2] = {zero, zero}, e1y[2] = {zero, zero}, e1z[2] = {zero, zero};
+  T az[2] = {zero, zero}, ax[2] = {zero, zero}, ay[2] = {zero, zero};
+  T e2x = zero, e2y = zero;
   __syncthreads();
+  // conductivity of level k: the lane's, the left neighbour's, the row above's, and its sums with the first
+  T sg = sg0, sl = from_left(sg0), su = sS[0][lym][lx], sp = sl + sg0, sq = su + sg0;
   __builtin_amdgcn_s_waitcnt(0);
 
-  auto level = [&](const int k, const LvT &cur, const LvT &nxt, LvT &dst) {
-    const int kB = k + 2, p = k & 1;  // level k+2 has the parity of k
-    const bool aon = k >= klo, bon = kB <= N - 1;
-    const int kBc = min(kB, N - 1);
-    const T dzA = aon ? sZ[k] : zero, rdzA = sZ[N + k], rdz2A = sZ[2 * N + k];
-    const T dzB = bon ? sZ[kBc] : zero, rdzB = sZ[N + kBc], rdz2B = sZ[2 * N + kBc];
-    const unsigned offA = (unsigned)k * PSb + colb, offB = (unsigned)kBc * PSb + colb;
+  auto level = [&](auto par, const int k, const LvT &cur, const LvT &nxt, LvT &dst) {
+    constexpr int p = decltype(par)::value, q = p ^ 1;
+    const int kB = k + 2, kBc = min(kB, N - 1);
+    // step B's first two iterations (levels N+1, N) see zeros but for level N-1's B, which rdz2B leaves out;
+    // the zeros that they store in level N-1 the third replaces
+    const bool bon = kB <= N - 1;
+    const T dzA = sZ[k], rdzA = sZ[N + k], rdz2A = sZ[2 * N + k];
+    const T dzB = bon ? sZ[kBc] : zero, rdzB = sZ[N + kBc], rdz2B = bon ? sZ[2 * N + kBc] : zero;
+    const int offB = kBc * (int)PSb;
     // ---- P1
-    const T bx_k = cur.bx, by_k = cur.by, bx_m = nxt.bx, by_m = nxt.by;
-    T bzAk = zero, bzBk = zero;
-    if (rBzA) {
-      bzA.add(dzA * (((kX ? from_right(bx_k) : sBx[p][ly][lxp]) - bx_k) * rdx + (sBy[p][lyp][lx] - by_k) * rdy));
-      bzAk = bzA.val();
-    }
+    const T bx_k = cur.bx, by_k = cur.by, bx_m = nxt.bx, by_m = nxt.by, b1xk = b1x[p], b1yk = b1y[p];
+    if (k >= klo) bzA.add(dzA, div2(from_right(bx_k) - bx_k, rdx, sBy[p][lyp][lx] - by_k, rdy));
+    const T bzAk = bzA.val();
     sBzA[ly][lx] = bzAk;
-    if (rBzB) {
-      bzB.add(dzB * (((kX ? from_right(b1xc) : sB1x[p][ly][lxp]) - b1xc) * rdx + (sB1y[p][lyp][lx] - b1yc) * rdy));
-      bzBk = bzB.val();
-    }
+    bzB.add(dzB, div2(from_right(b1xk) - b1xk, rdx, sB1y[p][lyp][lx] - b1yk, rdy));
+    const T bzBk = bzB.val();
     sBzB[ly][lx] = bzBk;
-    const T sgm = stage(k - 1, nxt);  // the lane's conductivity of level k-1
+    const T sgm = stage(q, nxt);
     const T ezo = cur.ez, exo = cur.ex, eyo = cur.ey;
     dst = load(k - 1 - PF);
     __syncthreads();
-    // ---- P2: intermediate E of level k (step A), new E of level k+2 (step B).  The conductivity
-    // averages of a level are the same for both steps: step A forms them, step B takes them two
-    // iterations later from registers.
-    T ezA = zero, exA = zero, eyA = zero, azA = zero, axA = zero, ayA = zero;
-    if (ezrow) {
-      const int sp = k & 1, sq = sp ^ 1;
-      const T sgkL = from_left(sgk), sgmL = from_left(sgm);
-      azA = (T)0.25 * (sS[sp][lym][lxm] + sS[sp][lym][lx] + sgkL + sgk);
-      {
-        const T sxk = (T)0.5 * (sS[sp][lym][lx] + sgk);
-        const T sxm = (T)0.5 * (sS[sq][lym][lx] + sgm);
-        axA = (T)0.5 * (sxk + sxm);
-      }
-      ayA = (T)0.25 * (sgkL + sgk + sgmL + sgm);
-      {
-        const T curl = (by_k - (kX ? from_left(by_k) : sBy[p][ly][lxm])) * rdx2 - (bx_k - sBx[p][lym][lx]) * rdy2;
-        const T v = df_new(ezo, azA, cfA, curl);
-        ezA = dEz ? v : zero;
-      }
-      if (rA) {
-        {
-          const T curl = (bzAk - sBzA[lym][lx]) * rdy2 - (by_k - by_m) * rdz2A;
-          const T v = df_new(exo, axA, cfA, curl);
-          exA = dEx ? v : zero;
-        }
-        {
-          const T curl = (bx_k - bx_m) * rdz2A - (bzAk - (kX ? from_left(bzAk) : sBzA[ly][lxm])) * rdx2;
-          const T v = df_new(eyo, ayA, cfA, curl);
-          eyA = dEy ? v : zero;
-        }
-      }
-    }
+    // ---- P2: intermediate E of level k (step A), new E of level k+2 (step B, the conductivity sums that step A
+    // formed two iterations earlier)
+    const T sum = sS[q][lym][lx], slm = from_left(sgm), spm = slm + sgm, sqm = sum + sgm;
+    const T azA = from_left(su) + su + sl + sg, axA = sq + sqm, ayA = sp + slm + sgm;
+    const T ezA = df_new(ezo, azA, cfA, curl2(by_k - from_left(by_k), zx, bx_k - sBx[p][lym][lx], zy));
     sEzA[ly][lx] = ezA;
+    const T exA = df_new(exo, axA, cfA, curl2(bzAk - sBzA[lym][lx], rdy2, by_k - by_m, rdz2A));
+    const T eyA = df_new(eyo, ayA, cfA, curl2(bx_k - bx_m, rdz2A, bzAk - from_left(bzAk), rdx2));
     T ezB = zero, exB = zero, eyB = zero;
-    if (rEzB) {
-      {
-        const T curl = (b1yc - (kX ? from_left(b1yc) : sB1y[p][ly][lxm])) * rdx2 - (b1xc - sB1x[p][lym][lx]) * rdy2;
-        const T v = df_new(e1zc, azc, cfB, curl);
-        ezB = bon && dEz ? v : zero;
-      }
-      if (rB) {
-        {
-          const T curl = (bzBk - sBzB[lym][lx]) * rdy2 - (b1yc - b1yn) * rdz2B;
-          const T v = df_new(e1xc, axc, cfB, curl);
-          exB = bon && dEx ? v : zero;
-        }
-        {
-          const T curl = (b1xc - b1xn) * rdz2B - (bzBk - (kX ? from_left(bzBk) : sBzB[ly][lxm])) * rdx2;
-          const T v = df_new(e1yc, ayc, cfB, curl);
-          eyB = bon && dEy ? v : zero;
-        }
-      }
+    if (rB) {
+      ezB = df_new(e1z[p], az[p], cfB, curl2(b1yk - from_left(b1yk), zx, b1xk - sB1x[p][lym][lx], zy));
+      exB = df_new(e1x[p], ax[p], cfB, curl2(bzBk - sBzB[lym][lx], rdy2, b1yk - b1y[q], rdz2B));
+      eyB = df_new(e1y[p], ay[p], cfB, curl2(b1xk - b1x[q], rdz2B, bzBk - from_left(bzBk), rdx2));
     }
     sEzB[ly][lx] = ezB;
-    const bool stB = own && bon;
-    bsto(rez, offB, stB && dEz, ezB);
-    bsto(rex, offB, stB && dEx, exB);
-    bsto(rey, offB, stB && dEy, eyB);
+    bsto_at<kSt>(rez, sEzo, offB, ezB);
+    bsto_at<kSt>(rex, sEx, offB, exB);
+    bsto_at<kSt>(rey, sEy, offB, eyB);
     __syncthreads();
-    // ---- P3: intermediate B of level k (step A, into LDS), new B of level k+2 (step B)
-    T b1xA = zero, b1yA = zero;
-    if (rA) {
-      const T bxA = bx_k + dtbA * ((e1yn - eyA) * rdzA - (sEzA[lyp][lx] - ezA) * rdy);
-      const T byA = by_k + dtbA * (((kX ? from_right(ezA) : sEzA[ly][lxp]) - ezA) * rdx - (e1xn - exA) * rdzA);
-      b1xA = dBx ? bxA : zero;
-      b1yA = dBy ? byA : zero;
-    }
-    sB1x[p][ly][lx] = b1xA;
-    sB1y[p][ly][lx] = b1yA;
-    const bool stA = own && k == klo;  // level 2 of the intermediate state, for the top launches
-    bsto(mex, offA, stA && dEx, exA);
-    bsto(mey, offA, stA && dEy, eyA);
-    bsto(mez, offA, stA && dEz, ezA);
-    bsto(mbx, offA, stA && dBx, b1xA);
-    bsto(mby, offA, stA && dBy, b1yA);
-    if (rB) {
-      const T bxB = b1xc + dtbB * ((e2y - eyB) * rdzB - (sEzB[lyp][lx] - ezB) * rdy);
-      const T byB = b1yc + dtbB * (((kX ? from_right(ezB) : sEzB[ly][lxp]) - ezB) * rdx - (e2x - exB) * rdzB);
-      bsto(rbx, offB, stB && dBx, bxB);
-      bsto(rby, offB, stB && dBy, byB);
+    // ---- P3: intermediate B of level k (step A, into LDS for step B), new B of level k+2 (step B)
+    const T bxv = fma_(dtbA, curl2(e1y[q] - eyA, rdzA, sEzA[lyp][lx] - ezA, rdy), bx_k);
+    const T byv = fma_(dtbA, curl2(from_right(ezA) - ezA, rdx, e1x[q] - exA, rdzA), by_k);
+    const T bxA = dEy ? bxv : zero, byA = dEx ? byv : zero;  // Bx has Ey's cells, By Ex's
+    sB1x[p][ly][lx] = bxA;
+    sB1y[p][ly][lx] = byA;
+    const T bxB = fma_(dtbB, curl2(e2y - eyB, rdzB, sEzB[lyp][lx] - ezB, rdy), b1xk);
+    const T byB = fma_(dtbB, curl2(from_right(ezB) - ezB, rdx, e2x - exB, rdzB), b1yk);
+    bsto_at<kSt>(rbx, sEy, offB, bxB);
+    bsto_at<kSt>(rby, sEx, offB, byB);
+    if (k == klo) {  // level 2 of the intermediate state, for the top launches
+      const int offA = k * (int)PSb;
+      bsto_at<kSt>(rsrc_of(pa.mex + fo, fbytes), sEx, offA, exA);
+      bsto_at<kSt>(rsrc_of(pa.mey + fo, fbytes), sEy, offA, eyA);
+      bsto_at<kSt>(rsrc_of(pa.mez + fo, fbytes), sEzo, offA, ezA);
+      bsto_at<kSt>(rsrc_of(pa.mbx + fo, fbytes), sEy, offA, bxA);
+      bsto_at<kSt>(rsrc_of(pa.mby + fo, fbytes), sEx, offA, byA);
     }
     e2x = exB;
     e2y = eyB;
-    b1xc = b1xn;
-    b1yc = b1yn;
-    b1xn = b1xA;
-    b1yn = b1yA;
-    e1xc = e1xn;
-    e1yc = e1yn;
-    e1zc = e1zn;
-    e1xn = exA;
-    e1yn = eyA;
-    e1zn = ezA;
-    azc = azn;
-    axc = axn;
-    ayc = ayn;
-    azn = azA;
-    axn = axA;
-    ayn = ayA;
-    sgk = sgm;
+    b1x[p] = bxA;
+    b1y[p] = byA;
+    e1x[p] = exA;
+    e1y[p] = eyA;
+    e1z[p] = ezA;
+    az[p] = azA;
+    ax[p] = axA;
+    ay[p] = ayA;
+    sg = sgm;
+    sl = slm;
+    su = sum;
+    sp = spm;
+    sq = sqm;
     // no barrier here: the next iteration's first phase writes only the Bz sums and the staging
     // buffers of level k-2, which no wave reads after this iteration's second barrier, and reads
     // the intermediate B of level k+1, which this phase does not write
   };
+  // unrolled by the ring and by the parity, so that every value keeps its registers and LDS its offsets
+  constexpr int U = S % 2 ? 2 * S : S;
   int k = khi;
-  for (; k - (S - 1) >= 1; k -= S) {
-#pragma unroll
-    for (int u = 0; u < S; ++u) level(k - u, R[u], R[(u + 1) % S], R[(u + S - 1) % S]);
+  for (; k - (U - 1) >= 1; k -= U) {
+    unrolled<U>([&](auto u) {
+      constexpr int v = decltype(u)::value;
+      level(std::integral_constant<int, v % 2>{}, k - v, R[v % S], R[(v + 1) % S], R[(v + S - 1) % S]);
+    });
   }
-#pragma unroll
-  for (int u = 0; u < S - 1; ++u)
-    if (k - u >= 1) level(k - u, R[u], R[(u + 1) % S], R[(u + S - 1) % S]);
+  unrolled<U - 1>([&](auto u) {
+    constexpr int v = decltype(u)::value;
+    if (k - v >= 1) level(std::integral_constant<int, v % 2>{}, k - v, R[v % S], R[(v + 1) % S], R[(v + S - 1) % S]);
+  });
   // the running sums for the top launches: step A's through level 2, step B's through level 3
   if (own && xin && yin) {
     bzA.save(a.cs + po, a.cc + po, colb);
@@ -957,32 +953,29 @@ __global__ void __launch_bounds__(kMarchLanes *BY) k_surface(const MarchArgs<T> 
   __syncthreads();
   T ezn;
   {
-    const T s4 = (T)0.25 * (sS[lym][lxm] + sS[lym][lx] + sS[ly][lxm] + sS[ly][lx]);
-    const T curl = (by0 - sBy[ly][lxm]) * rdx2 - (bx0 - sBx[lym][lx]) * rdy2;
+    const T s4 = sS[lym][lxm] + sS[lym][lx] + sS[ly][lxm] + sS[ly][lx];
+    const T curl = curl2(by0 - sBy[ly][lxm], rdx2, bx0 - sBx[lym][lx], rdy2);
     ezn = apply_src(df_new(ezo, s4, cf, curl), 2, 0, j, i, a, sfirst, scount);
     ezn = ln.vEzAny ? ezn : zero;
   }
   sEz[ly][lx] = ezn;
   if (ln.vEz) sto(ez, off, ezn);
   T exn, eyn;
-  {
-    const T sxk = (T)0.5 * (sS[lym][lx] + sS[ly][lx]);
-    const T ave = (T)0.5 * (sxk + zero);
-    const T curl = (bzc - sBz[lym][lx]) * rdy2 - (by0 - bya) * rdz20;
-    exn = apply_src(df_new(exo, ave, cf, curl), 0, 0, j, i, a, sfirst, scount);
+  {  // no conductivity above the sea surface: two cells of the four
+    const T curl = curl2(bzc - sBz[lym][lx], rdy2, by0 - bya, rdz20);
+    exn = apply_src(df_new(exo, sS[lym][lx] + sS[ly][lx], cf, curl), 0, 0, j, i, a, sfirst, scount);
     exn = ln.vEx ? exn : zero;
   }
   {
-    const T s4 = (T)0.25 * (sS[ly][lxm] + sS[ly][lx]);
-    const T curl = (bx0 - bxa) * rdz20 - (bzc - sBz[ly][lxm]) * rdx2;
-    eyn = apply_src(df_new(eyo, s4, cf, curl), 1, 0, j, i, a, sfirst, scount);
+    const T curl = curl2(bx0 - bxa, rdz20, bzc - sBz[ly][lxm], rdx2);
+    eyn = apply_src(df_new(eyo, sS[ly][lxm] + sS[ly][lx], cf, curl), 1, 0, j, i, a, sfirst, scount);
     eyn = ln.vEy ? eyn : zero;
   }
   if (ln.vEx) sto(ex, off, exn);
   if (ln.vEy) sto(ey, off, eyn);
   __syncthreads();
-  const T bxn = bx0 + dtb * ((ey1 - eyn) * rdz0 - (sEz[lyp][lx] - ezn) * rdy);
-  const T byn = by0 + dtb * ((sEz[ly][lxp] - ezn) * rdx - (ex1 - exn) * rdz0);
+  const T bxn = fma_(dtb, curl2(ey1 - eyn, rdz0, sEz[lyp][lx] - ezn, rdy), bx0);
+  const T byn = fma_(dtb, curl2(sEz[ly][lxp] - ezn, rdx, ex1 - exn, rdz0), by0);
   if (ln.vBx) sto(bx, off, bxn);
   if (ln.vBy) sto(by, off, byn);
 }
@@ -1034,11 +1027,11 @@ __global__ void __launch_bounds__(256) k_src(const MarchArgs<T> la, const MarchA
       T old, nw;
       if (sc.comp == 3) {
         old = bx[o];
-        nw = bxi[o] + dtb * ((ey[o + PS] - ey[o]) * rdzk - (ez[o + PX] - ez[o]) * a.rdy[sc.j + 1]);
+        nw = fma_(dtb, curl2(ey[o + PS] - ey[o], rdzk, ez[o + PX] - ez[o], a.rdy[sc.j + 1]), bxi[o]);
         bx[o] = nw;
       } else {
         old = by[o];
-        nw = byi[o] + dtb * ((ez[o + 1] - ez[o]) * a.rdx[sc.i + 1] - (ex[o + PS] - ex[o]) * rdzk);
+        nw = fma_(dtb, curl2(ez[o + 1] - ez[o], a.rdx[sc.i + 1], ex[o + PS] - ex[o], rdzk), byi[o]);
         by[o] = nw;
       }
       if (a.ibw && sc.k >= 2) {  // levels 2 .. N-1 belong to the lower launch's chunks
@@ -1070,7 +1063,7 @@ __global__ void __launch_bounds__(256) k_zsum(const MarchArgs<T> a) {
 #pragma unroll 4
   for (int k = hi; k >= lo; --k) {
     const long long o = (long long)k * a.PS;
-    acc.add(a.dzt[k] * ((bx[o + 1] - bx[o]) * rdx + (by[o + a.PX] - by[o]) * rdy));
+    acc.add(a.dzt[k], div2(bx[o + 1] - bx[o], rdx, by[o + a.PX] - by[o], rdy));
   }
   a.zs[c * a.zstride + (long long)slot * a.pstride + (long long)j * a.PX + i] = acc.val();
 }
@@ -1090,7 +1083,7 @@ __global__ void k_bz_volume(const MarchArgs<T> a, T *bzout, int slot) {
   bzout[((long long)N * M + j) * L + i] = 0;
   for (int k = N - 1; k >= 0; --k) {
     const long long o = (long long)k * a.PS + (long long)j * a.PX + i;
-    acc.add(a.dzt[k] * ((bx[o + 1] - bx[o]) * rdx + (by[o + a.PX] - by[o]) * rdy));
+    acc.add(a.dzt[k], div2(bx[o + 1] - bx[o], rdx, by[o + a.PX] - by[o], rdy));
     bzout[((long long)k * M + j) * L + i] = acc.val();
   }
 }
@@ -1157,11 +1150,11 @@ __global__ void __launch_bounds__(kGatherThreads) k_gather(const GatherArgs g, c
     const long long base = (long long)jj * g.PX + ii;
     auto div = [&](int k) {
       const long long o = (long long)k * g.PS + base;
-      return (T)(a.dzt[k] * ((bxf[o + 1] - bxf[o]) * rdx + (byf[o + g.PX] - byf[o]) * rdy));
+      return div2(bxf[o + 1] - bxf[o], rdx, byf[o + g.PX] - byf[o], rdy);
     };
     Acc<T> acc;
     acc.init();
-    for (int k = g.N - 1 - part; k >= s3 + 4; k -= 16) acc.add(div(k));
+    for (int k = g.N - 1 - part; k >= s3 + 4; k -= 16) acc.add(a.dzt[k], div(k));
     spart[lane] = (double)acc.val();
     __syncthreads();
     if (part == 0) {
@@ -1169,7 +1162,7 @@ __global__ void __launch_bounds__(kGatherThreads) k_gather(const GatherArgs g, c
       for (int p = 15; p >= 0; --p) run += spart[col * 16 + p];
       for (int ik = 3; ik >= 0; --ik) {
         const int k = s3 + ik;
-        if (k < g.N) run += (double)div(k);
+        if (k < g.N) run += (double)(a.dzt[k] * div(k));
         sv[ik * 16 + ij * 4 + q] = k < g.N ? run : 0.0;
       }
     }
