@@ -477,6 +477,7 @@ struct tcsem_ctx {
   int2 *d_fixg = nullptr;
   int *d_fixidx = nullptr;  // E first[nbatch], E count[nbatch], run first[nbatch], run count[nbatch]
   bool has_fix = false;
+  int fix_kmin = 0;  // lowest level of d_fixe
   int *d_rxl = nullptr;     // rx_local, rx_first[nbatch], rx_count[nbatch]
   int *d_ops = nullptr;     // it of every op of the run (E ops then B ops)
   double *d_opl1 = nullptr;
@@ -1282,16 +1283,18 @@ hipError_t enqueue_march(tcsem_ctx *c, const MarchArgs<T> &a, int nb, hipStream_
   return launch_march<T>(hi, nb, st, te[2], te[3]);
 }
 
+// The source's amplitude at step n (main.cu:223-252): zero past the wavelet.
+double source_amp(const tcsem_ctx *c, int n) { return n < 2 * (c->setup.n_src / 2) ? c->wwave[n] : 0.0; }
+
 // Step scalars of the context's current step (main.cu:223-260).
 template <typename T>
 void step_scalars(const tcsem_ctx *c, MarchArgs<T> &a) {
   const tcsem_setup &s = c->setup;
-  const int ns = s.n_src / 2;
   const double mindx = c->g.mindx;
   a.lam = 7.5 * s.sfa2 * c->dt2 * c->dt1 / kMu0 / mindx / mindx;  // main.cu:223
   a.dt = c->dt1;
   a.dtb = 0.5 * (c->dt1 + c->dt2);
-  a.amp = c->n < 2 * ns ? c->wwave[c->n] : 0.0;
+  a.amp = source_amp(c, c->n);
 }
 
 // Time advance after a step (main.cu:253-260).
@@ -1413,6 +1416,7 @@ int do_step(tcsem_ctx *c) {
     sp.fixg = c->d_fixg;
     sp.fixidx = c->d_fixidx;
     sp.fixn = nb;
+    sp.fixtop = N - 1;
     if (split && c->nchunk > 1 && c->fuse) {
       sp.ibw = ib_planes(c, c->ib_par);  // the parity this step's lower launch wrote
       sp.ibstride = (long long)c->nslots * c->pstride;
@@ -1593,12 +1597,14 @@ int graph_steps(tcsem_ctx *c) {
 // go to stream2 and overlap the next pass.  The pass reads the old state at levels >= 1 only and
 // writes the intermediate state at level 2 only, so it too runs beside the previous step's
 // stream2 work.
-// Whether the next two steps may run as a pair: pairs on, past the source (no amplitude, no source
-// pass), and no receiver sample after the first of them (one after the second is taken from the
-// new state as usual).
+// The source cells of a source step are patched in the pass itself (levels 2 up for step A, 3 up for step B);
+// those above are patched after each top launch, as after a single step's march (when source steps ran one
+// at a time, 220 x 200 x 110 FP64 over 40 source steps of 60 took 21.5 ms against 19.0 in pairs, 256 x 256 x 160 FP64
+// over 100 of 500 93 against 82 ms, 512 x 512 x 256 FP32 over 40 of 400 180 against 173 ms).
+// Whether the next two steps may run as a pair: pairs on, and no receiver sample after the first of them
+// (one after the second is taken from the new state as usual).
 bool pair_ok(tcsem_ctx *c, long room) {
-  return c->pair_by > 0 && room >= 2 && c->g.info.N >= 6 && c->n >= 2 * (c->setup.n_src / 2) &&
-         !events_ahead(c, 1);
+  return c->pair_by > 0 && room >= 2 && c->g.info.N >= 6 && !events_ahead(c, 1);
 }
 
 hipError_t ensure_mid(tcsem_ctx *c) {
@@ -1627,7 +1633,15 @@ hipError_t enqueue_pair(tcsem_ctx *c, const MarchArgs<T> &a, const MarchArgs<T> 
   const long long org = c->PX + c->xm, fs = c->fstride * c->nslots, ps = c->pstride * c->nslots;
   T *fm = (T *)c->d_mid, *pl = (T *)c->d_planes;
   PairArgs<T> p{};
-  p.a = a;
+  MarchArgs<T> sa = a;
+  if (c->has_fix) {
+    sa.fixe = c->d_fixe;
+    sa.fixb = c->d_fixb;
+    sa.fixg = c->d_fixg;
+    sa.fixidx = c->d_fixidx;
+    sa.fixn = nb;
+  }
+  p.a = sa;
   p.a.pf = c->pair_pf;
   p.mex = fm + org;
   p.mey = fm + fs + org;
@@ -1639,12 +1653,15 @@ hipError_t enqueue_pair(tcsem_ctx *c, const MarchArgs<T> &a, const MarchArgs<T> 
   p.lamB = sb.lam;
   p.dtB = sb.dt;
   p.dtbB = sb.dtb;
+  p.ampB = sb.amp;
+  p.src = c->has_fix && (sa.amp != 0.0 || sb.amp != 0.0);
   p.rows = c->pair_by;
   p.ntx = c->pair_ntx;
   p.nty = c->pair_nty;
   p.nper = c->pair_nper;
   // top launch and surface of step A: old state -> intermediate state
-  MarchArgs<T> ta = a;
+  MarchArgs<T> ta = sa;
+  ta.fixtop = 1;
   ta.ex = p.mex;
   ta.ey = p.mey;
   ta.ez = p.mez;
@@ -1653,7 +1670,8 @@ hipError_t enqueue_pair(tcsem_ctx *c, const MarchArgs<T> &a, const MarchArgs<T> 
   ta.k_hi = 1;
   ta.carry = 1;
   // top launch (levels 2, 1) and surface of step B: intermediate state -> new state
-  MarchArgs<T> tb = a;
+  MarchArgs<T> tb = sa;
+  tb.fixtop = 2;
   tb.exi = p.mex;
   tb.eyi = p.mey;
   tb.ezi = p.mez;
@@ -1662,7 +1680,7 @@ hipError_t enqueue_pair(tcsem_ctx *c, const MarchArgs<T> &a, const MarchArgs<T> 
   tb.lam = sb.lam;
   tb.dt = sb.dt;
   tb.dtb = sb.dtb;
-  tb.amp = 0.0;
+  tb.amp = sb.amp;
   tb.k_hi = 2;
   tb.carry = 1;
   tb.cs = p.cs2;
@@ -1670,9 +1688,11 @@ hipError_t enqueue_pair(tcsem_ctx *c, const MarchArgs<T> &a, const MarchArgs<T> 
   if ((e = launch_march2<T>(p, nb, st, te[0], te[1])) != hipSuccess) return e;
   if ((e = hipStreamWaitEvent(st, c->xev[1], 0)) != hipSuccess) return e;  // the previous step's stream2 work
   if ((e = launch_march<T>(ta, nb, st, te[2], te[3])) != hipSuccess) return e;
+  if (p.src && ta.amp != 0.0 && c->fix_kmin <= 1 && (e = launch_src<T>(ta, nb, st)) != hipSuccess) return e;
   if ((e = launch_upcont<T>(u, nb, st, te[4], te[5], nullptr, true)) != hipSuccess) return e;
   if ((e = launch_surface<T>(ta, nb, st, te[6], te[7])) != hipSuccess) return e;
   if ((e = launch_march<T>(tb, nb, st, te[8], te[9])) != hipSuccess) return e;
+  if (p.src && tb.amp != 0.0 && c->fix_kmin <= 2 && (e = launch_src<T>(tb, nb, st)) != hipSuccess) return e;
   if ((e = hipEventRecord(c->xev[0], st)) != hipSuccess) return e;
   if ((e = hipStreamWaitEvent(st2, c->xev[0], 0)) != hipSuccess) return e;
   if ((e = launch_upcont<T>(u, nb, st2, te[10], te[11])) != hipSuccess) return e;
@@ -2239,6 +2259,15 @@ int batch_quiesce(tcsem_batch *b) {
   return batch_collect(b);
 }
 
+// Whether an active member's source acts `ahead` steps from now on cells at levels 1 .. top.
+bool batch_source(const tcsem_batch *b, int ahead, int top) {
+  for (size_t q = 0; q < b->m.size(); ++q) {
+    const tcsem_ctx *c = b->m[q];
+    if (b->active[q] && c->has_fix && c->fix_kmin <= top && source_amp(c, c->n + ahead) != 0.0) return true;
+  }
+  return false;
+}
+
 // One batch step on the batch's streams, as do_step for one context: lower march of every member,
 // (after the previous step's stream2 work) the top march, the members' source pass; on stream2
 // the air-plane chain, the surface level and the members' receiver gathers.  par: record parity.
@@ -2271,16 +2300,10 @@ int batch_enqueue(tcsem_batch *b, const MarchArgs<T> &la, const UpcontArgs<T> &u
   HIPCHK(launch_march<T>(lo, 1, st, te[0], te[1], geo));  // one grid row: the work list
   HIPCHK(hipStreamWaitEvent(st, b->xev[1], 0));
   HIPCHK(launch_march<T>(hi, 1, st, te[2], te[3], geo));
-  if (live) {  // one source pass for every member with a source cell this step
-    bool src = false;
-    for (int q = 0; q < nm && !src; ++q) {
-      tcsem_ctx *c = b->m[q];
-      if (!b->active[q] || !c->has_fix) continue;
-      MarchArgs<T> a{};
-      step_scalars<T>(c, a);
-      src = a.amp != 0.0;
-    }
-    if (src) HIPCHK(launch_src<T>(hi, nm, st, geo));
+  if (live && batch_source(b, 0, la.N - 1)) {  // one source pass for every member with a source cell this step
+    MarchArgs<T> sp = hi;
+    sp.fixtop = la.N - 1;
+    HIPCHK(launch_src<T>(sp, nm, st, geo));
   }
   HIPCHK(hipEventRecord(b->xev[0], st));
   HIPCHK(hipStreamWaitEvent(st2, b->xev[0], 0));
@@ -2324,13 +2347,16 @@ int batch_enqueue_pair(tcsem_batch *b, const MarchArgs<T> &la, const UpcontArgs<
   pl.gscalB = b->d_scal + (size_t)(row + 1) * nm * 4;
   pl.rows = b->pair_by;
   pl.nper = b->pwork_len / 8;
+  pl.src = live && (batch_source(b, 0, la.N - 1) || batch_source(b, 1, la.N - 1));
   MarchArgs<T> ta = la, tb = la;
   ta.gscal = pl.a.gscal;
   tb.gscal = pl.gscalB;
   ta.k_hi = 1;
   ta.k_lo = 1;
   ta.carry = 1;
+  ta.fixtop = 1;
   tb.k_hi = 2;
+  tb.fixtop = 2;
   tb.k_lo = 1;
   tb.carry = 1;
   const bool timed = b->timing && (b->nenq % kTimingStride == 0 || (b->nenq + 1) % kTimingStride == 0);
@@ -2348,9 +2374,11 @@ int batch_enqueue_pair(tcsem_batch *b, const MarchArgs<T> &la, const UpcontArgs<
   HIPCHK(launch_march2<T>(pl, 1, st, te[0], te[1], pg));
   HIPCHK(hipStreamWaitEvent(st, b->xev[1], 0));
   HIPCHK(launch_march<T>(ta, 1, st, te[2], te[3], tga));
+  if (live && batch_source(b, 0, 1)) HIPCHK(launch_src<T>(ta, nm, st, tga));
   HIPCHK(launch_upcont<T>(ul, nm, st, te[4], te[5], ugeo, true));
   HIPCHK(launch_surface<T>(ta, nm, st, te[6], te[7], tga));
   HIPCHK(launch_march<T>(tb, 1, st, te[8], te[9], tgb));
+  if (live && batch_source(b, 1, 2)) HIPCHK(launch_src<T>(tb, nm, st, tgb));
   HIPCHK(hipEventRecord(b->xev[0], st));
   HIPCHK(hipStreamWaitEvent(st2, b->xev[0], 0));
   HIPCHK(launch_upcont<T>(ul, nm, st2, te[10], te[11], ugeo));
@@ -2381,13 +2409,11 @@ int batch_enqueue_pair(tcsem_batch *b, const MarchArgs<T> &la, const UpcontArgs<
   return TCSEM_OK;
 }
 
-// Whether the batch's next two steps may run as a pair: every member still sampling is past its
-// source wavelet and takes no receiver sample after the first of the two steps.
+// Whether the batch's next two steps may run as a pair: no member still sampling takes a receiver sample
+// after the first of them.
 bool batch_pair_ok(tcsem_batch *b) {
   for (size_t q = 0; q < b->m.size(); ++q) {
-    if (!b->active[q]) continue;
-    tcsem_ctx *c = b->m[q];
-    if (c->n < 2 * (c->setup.n_src / 2) || events_ahead(c, 1)) return false;
+    if (b->active[q] && events_ahead(b->m[q], 1)) return false;
   }
   return true;
 }
@@ -3415,7 +3441,7 @@ int tcsem_reset_fields(tcsem_ctx *c, int first, int n) {
 // slot's table once, with the weights of coincident entries summed in table order (the order of
 // the per-cell loop of ElectricalFiled.cu:347-475), then every Bx/By cell whose curl reads one of
 // them (Bderivate.cu:79-200), sorted by (component, j, i, k) and cut into one run per component
-// and column.  Cells outside the update masks are dropped, as the march drops them; level-0 cells
+// and column; the E cells by level.  Cells outside the update masks are dropped, as the march drops them; level-0 cells
 // stay with the surface kernel.
 static int build_fix_lists(tcsem_ctx *c, int nbatch) {
   const int L = c->g.info.L, M = c->g.info.M, N = c->g.info.N;
@@ -3433,6 +3459,7 @@ static int build_fix_lists(tcsem_ctx *c, int nbatch) {
   std::vector<SrcCell> ecells, bcells;
   std::vector<int2> runs;
   std::vector<int> idx(4 * nbatch, 0);
+  c->fix_kmin = N;
   for (int b = 0; b < nbatch; ++b) {
     idx[b] = (int)ecells.size();
     idx[2 * nbatch + b] = (int)runs.size();
@@ -3481,6 +3508,8 @@ static int build_fix_lists(tcsem_ctx *c, int nbatch) {
         if (x.i != y.i) return x.i < y.i;
         return x.k < y.k;
       });
+      std::sort(ecells.begin() + e0, ecells.end(), [](const SrcCell &x, const SrcCell &y) { return x.k < y.k; });
+      if (ecells.size() > e0) c->fix_kmin = std::min(c->fix_kmin, ecells[e0].k);
       for (size_t q = b0; q < bcells.size(); ++q) {
         const SrcCell &x = bcells[q];
         const bool same = q > b0 && bcells[q - 1].comp == x.comp && bcells[q - 1].j == x.j && bcells[q - 1].i == x.i;

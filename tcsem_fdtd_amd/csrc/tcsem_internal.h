@@ -111,11 +111,12 @@ struct MarchArgs {
   // once, the weights of coincident table entries summed) fixe[fixidx[s] ..] (count
   // fixidx[fixn + s]), and the Bx/By cells whose curl reads one of them, grouped by column:
   // fixg[fixidx[2 fixn + s] ..] (count fixidx[3 fixn + s]) holds (first, count) runs of fixb, one
-  // run per (component, j, i), levels ascending.  Null fixe: no source pass.
+  // run per (component, j, i), levels ascending.  Null fixe: no source pass.  fixe's levels ascend.
+  // fixtop: the source pass takes cells at levels up to this one (the two-step pass has taken the others)
   const SrcCell *fixe, *fixb;
   const int2 *fixg;
   const int *fixidx;
-  int fixn;
+  int fixn, fixtop;
 };
 
 // Two steps in one lower pass (k_march2): step A advances the old state (a.exi ..) to the
@@ -131,8 +132,9 @@ struct PairArgs {
   MarchArgs<T> a;                  // step A's scalars; old and new state; carry planes of step A
   T *mex, *mey, *mez, *mbx, *mby;  // intermediate state (origin, slot 0)
   T *cs2, *cc2;                    // carry planes of step B (plane origin, slot 0)
-  double lamB, dtB, dtbB;          // step B's scalars
+  double lamB, dtB, dtbB, ampB;    // step B's scalars
   int rows, ntx, nty, nper;
+  int src;                         // launch record: a source acts in either step
   const double *gscalB;            // model batch, launch record only: step B's row of the scalar table
 };
 

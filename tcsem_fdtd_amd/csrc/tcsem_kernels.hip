@@ -18,8 +18,8 @@
 // Level 0 needs the air fields from the upward continuation of Bz(0), so the march stops at
 // level 1 and writes Bz_old(0); k_surface finishes level 0 after the air planes are ready.
 //
-// Two-step pass (k_march2): on steady-state steps two consecutive steps share one bottom-up pass
-// over levels N-1 .. 3, the second step two levels behind the first, so the state between them
+// Two-step pass (k_march2): two consecutive steps (no receiver sample between them) share one bottom-up
+// pass over levels N-1 .. 3, the second step two levels behind the first, so the state between them
 // stays in registers and LDS; the top levels of both steps run through k_march and k_surface.
 #include <type_traits>
 
@@ -303,6 +303,7 @@ __device__ inline MarchArgs<T> slot_args(const MarchArgs<T> &la, const MarchArgs
   if (la.carry == 1) a.k_hi = la.k_hi;  // the top launch: level 1; the lower launch: N-1 of the slot
   a.nchunk = 0;
   a.chunk_len = 0;
+  a.fixtop = la.fixtop;
   return a;
 }
 
@@ -673,7 +674,9 @@ struct Lv2 {
 // GEO: a model batch, one record per member (its fields, tables, sizes, intermediate state, carry
 // planes and pass tiles) and a 1-D grid over the launch's work list of (member, tile) pairs; the
 // launch record la carries the work list and both steps' scalar tables.
-template <typename T, int BY, int PF, bool S8, bool GEO>
+// SRC: a source acts in either step; the steady state's variant carries none of it (with the source's scalars
+// and branches in it the pass ran 2.5 to 7% slower).
+template <typename T, int BY, int PF, bool S8, bool GEO, bool SRC>
 __global__ void __launch_bounds__(kMarchLanes *BY) k_march2(const PairArgs<T> la, const PairArgs<T> *geo) {
   PairArgs<T> pa;
   int tile;
@@ -688,6 +691,8 @@ __global__ void __launch_bounds__(kMarchLanes *BY) k_march2(const PairArgs<T> la
     pa.lamB = qb[0];
     pa.dtB = qb[1];
     pa.dtbB = qb[2];
+    pa.a.amp = qa[3];
+    pa.ampB = qb[3];
     tile = w.y;
   } else {
     pa = la;
@@ -800,6 +805,43 @@ __global__ void __launch_bounds__(kMarchLanes *BY) k_march2(const PairArgs<T> la
   T e1x[2] = {zero, zero}, e1y[2] = {zero, zero}, e1z[2] = {zero, zero};
   T az[2] = {zero, zero}, ax[2] = {zero, zero}, ay[2] = {zero, zero};
   T e2x = zero, e2y = zero;
+  // Source cells of both steps (ElectricalFiled.cu:347-475; fixe, levels ascending): the next cell of each step
+  // and its level (-1: none left, or none in this wave's row of the tile)
+  const SrcCell *fixe = nullptr;
+  int srcA = -1, srcB = -1, kSrcA = -1, kSrcB = -1;
+  if (SRC && a.fixe && (a.amp != 0.0 || pa.ampB != 0.0)) {
+    const int ne = a.fixidx[a.fixn + slot];
+    fixe = a.fixe + a.fixidx[slot];
+    bool hit = false;
+    for (int q = lx; q < ne; q += W) hit = hit || (fixe[q].j == j && (unsigned)(fixe[q].i - (i - lx)) < (unsigned)W);
+    if (__any(hit)) {
+      if (a.amp != 0.0) srcA = ne - 1;
+      if (pa.ampB != 0.0) srcB = ne - 1;
+      if (srcA >= 0) kSrcA = fixe[srcA].k;
+      if (srcB >= 0) kSrcB = fixe[srcB].k;
+    }
+  }
+  // E - amp w of the cells at a level, 64 cells at a time
+  auto source = [&](const int lv, const double amp, int &at, int &lvl, T &ex, T &ey, T &ez) {
+    int n;
+    do {
+      const SrcCell sc = fixe[max(at - lx, 0)];
+      const bool here = lx <= at && sc.k == lv;
+      n = __popcll(__ballot(here));
+      for (unsigned long long m = __ballot(here && sc.j == j); m; m &= m - 1) {
+        const int b = __builtin_ctzll(m), comp = __builtin_amdgcn_readlane(sc.comp, b);
+        const unsigned long long wb = (unsigned long long)__double_as_longlong(sc.w);
+        const unsigned wl = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)wb, b);
+        const unsigned wh = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(wb >> 32), b);
+        const double w = __longlong_as_double((long long)(((unsigned long long)wh << 32) | wl));
+        if (__builtin_amdgcn_readlane(sc.i, b) != i) continue;
+        T &e = comp == 0 ? ex : comp == 1 ? ey : ez;
+        e = (T)((double)e - amp * w);
+      }
+      at -= n;
+    } while (n == W);
+    lvl = at >= 0 ? __builtin_amdgcn_readfirstlane(fixe[at].k) : -1;
+  };
   __syncthreads();
   // conductivity of level k: the lane's, the left neighbour's, the row above's, and its sums with the first
   T sg = sg0, sl = from_left(sg0), su = sS[0][lym][lx], sp = sl + sg0, sq = su + sg0;
@@ -830,16 +872,18 @@ __global__ void __launch_bounds__(kMarchLanes *BY) k_march2(const PairArgs<T> la
     // formed two iterations earlier)
     const T sum = sS[q][lym][lx], slm = from_left(sgm), spm = slm + sgm, sqm = sum + sgm;
     const T azA = from_left(su) + su + sl + sg, axA = sq + sqm, ayA = sp + slm + sgm;
-    const T ezA = df_new(ezo, azA, cfA, curl2(by_k - from_left(by_k), zx, bx_k - sBx[p][lym][lx], zy));
+    T ezA = df_new(ezo, azA, cfA, curl2(by_k - from_left(by_k), zx, bx_k - sBx[p][lym][lx], zy));
+    T exA = df_new(exo, axA, cfA, curl2(bzAk - sBzA[lym][lx], rdy2, by_k - by_m, rdz2A));
+    T eyA = df_new(eyo, ayA, cfA, curl2(bx_k - bx_m, rdz2A, bzAk - from_left(bzAk), rdx2));
+    if (SRC && k == kSrcA) source(k, a.amp, srcA, kSrcA, exA, eyA, ezA);
     sEzA[ly][lx] = ezA;
-    const T exA = df_new(exo, axA, cfA, curl2(bzAk - sBzA[lym][lx], rdy2, by_k - by_m, rdz2A));
-    const T eyA = df_new(eyo, ayA, cfA, curl2(bx_k - bx_m, rdz2A, bzAk - from_left(bzAk), rdx2));
     T ezB = zero, exB = zero, eyB = zero;
     if (rB) {
       ezB = df_new(e1z[p], az[p], cfB, curl2(b1yk - from_left(b1yk), zx, b1xk - sB1x[p][lym][lx], zy));
       exB = df_new(e1x[p], ax[p], cfB, curl2(bzBk - sBzB[lym][lx], rdy2, b1yk - b1y[q], rdz2B));
       eyB = df_new(e1y[p], ay[p], cfB, curl2(b1xk - b1x[q], rdz2B, bzBk - from_left(bzBk), rdx2));
     }
+    if (SRC && kB == kSrcB) source(kB, pa.ampB, srcB, kSrcB, exB, eyB, ezB);
     sEzB[ly][lx] = ezB;
     bsto_at<kSt>(rez, sEzo, offB, ezB);
     bsto_at<kSt>(rex, sEx, offB, exB);
@@ -1009,6 +1053,7 @@ __global__ void __launch_bounds__(256) k_src(const MarchArgs<T> la, const MarchA
   const int e0 = a.fixidx[s], ne = a.fixidx[n + s];
   for (int q = threadIdx.x; q < ne; q += blockDim.x) {
     const SrcCell sc = a.fixe[e0 + q];
+    if (sc.k > a.fixtop) continue;
     T *e = f[sc.comp] + (long long)sc.k * PS + (long long)sc.j * PX + sc.i;
     *e = (T)((double)*e - a.amp * sc.w);
   }
@@ -1022,6 +1067,7 @@ __global__ void __launch_bounds__(256) k_src(const MarchArgs<T> la, const MarchA
     const int2 run = a.fixg[g0 + g];
     for (int q = run.x; q < run.x + run.y; ++q) {
       const SrcCell sc = a.fixb[q];
+      if (sc.k > a.fixtop) break;  // a run's levels ascend
       const long long o = (long long)sc.k * PS + (long long)sc.j * PX + sc.i;
       const T rdzk = a.rdz[sc.k];
       T old, nw;
@@ -1267,19 +1313,22 @@ int pair_rows_supported(int prec, int rows) {
   if (prec == 32) return rows == 14 || rows == 16 ? rows : 0;
   return rows == 11 ? rows : 0;
 }
-template <typename T, int BY, int PF, bool S8, bool GEO>
+template <typename T, int BY, int PF, bool S8, bool GEO, bool SRC = false>
 hipError_t launch_march2_v(const PairArgs<T> &p, int nslot, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
                            const PairArgs<T> *geo) {
+  if constexpr (!SRC) {
+    if (p.src) return launch_march2_v<T, BY, PF, S8, GEO, true>(p, nslot, s, e0, e1, geo);
+  }
   const size_t zl = (size_t)3 * p.a.N * sizeof(T);
   static size_t allowed = 0;  // per instantiation; only grows
   if (zl > allowed) {
-    const hipError_t e = hipFuncSetAttribute((const void *)k_march2<T, BY, PF, S8, GEO>,
+    const hipError_t e = hipFuncSetAttribute((const void *)k_march2<T, BY, PF, S8, GEO, SRC>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)zl);
     if (e != hipSuccess) return e;
     allowed = zl;
   }
   dim3 blk(kMarchLanes, BY), grd(8 * p.nper, GEO ? 1 : nslot);
-  launch_k(k_march2<T, BY, PF, S8, GEO>, grd, blk, (std::uint32_t)zl, s, e0, e1, p, geo);
+  launch_k(k_march2<T, BY, PF, S8, GEO, SRC>, grd, blk, (std::uint32_t)zl, s, e0, e1, p, geo);
   return hipGetLastError();
 }
 template <typename T, int BY>
