@@ -179,8 +179,10 @@ __global__ void __launch_bounds__(1024) k_dn_y(const UpcontArgs<T> u0, const Upc
 }
 
 // ---- back to the irregular points: out[j][i] = sum_q R[q][j] b[q][i] -------------------------------
-// One workgroup per 32 x 16 tile of an air plane; its eight wavefronts share the sum over q.
-constexpr int kOutWaves = 8;
+// One workgroup per 32 x 16 tile of an air plane; its wavefronts share the sum over q.  A plane gives few tiles
+// (182 on 220 x 200) and the sum may be long (q < 3916 under 3914 regular columns), so latency bounds it: there 16
+// wavefronts with eight loads of a stream in flight take 42 us, 8 with four took 66; short sums are the same either way.
+constexpr int kOutWaves = 16;
 template <typename T, bool GEO>
 __global__ void __launch_bounds__(64 * kOutWaves) k_dn_out(const UpcontArgs<T> u0, const UpcontArgs<T> *geo) {
   const UpcontArgs<T> u = dense_record<GEO>(u0, geo);
@@ -193,7 +195,7 @@ __global__ void __launch_bounds__(64 * kOutWaves) k_dn_out(const UpcontArgs<T> u
   const double *R = (comp ? u.d.Ry : u.d.Rx) + (long long)slot * u.d.sP + j0 + r;
   const double *B = (comp ? u.d.by : u.d.bx) + i0 + r;
   d4 c0 = {}, c1 = {};
-#pragma unroll 4
+#pragma unroll 8
   for (int q = 4 * w + g; q < ((W2 + 3) & ~3); q += 4 * kOutWaves) {
     const long long o = (long long)min(q, W2 - 1) * MP;  // b has zero rows past W2
     const double b = B[(long long)q * ldb];
@@ -206,6 +208,7 @@ __global__ void __launch_bounds__(64 * kOutWaves) k_dn_out(const UpcontArgs<T> u
     red[w][16 + 4 * t + g][r] = c1[t];
   }
   __syncthreads();
+  if (threadIdx.x >= 512) return;
   const int j = threadIdx.x >> 4, i = threadIdx.x & 15;
   double v = red[0][j][i];
 #pragma unroll
