@@ -2423,9 +2423,7 @@ bool batch_pair_ok(tcsem_batch *b) {
 }
 
 // Rows of the batch's two-step passes: tcsem_batch_set_pairs' choice, else TCSEM_MARCH_PAIRS
-// ("0" or "rows[,1]"), else the autotuner's, else 12-row (FP64: 8-row) passes when the members'
-// pass tiles give at least two workgroups per CU (0: one step at a time); measured on the 64
-// uneven models, FP64 batches ran 6% faster with 8 rows than with 12.
+// ("0" or "rows[,1]"), else the autotuner's, else pass_rows over the members' tiles (0: one step at a time).
 int batch_pair_rows(tcsem_batch *b) {
   if (b->pair_set >= 0) return b->pair_set;
   if (const char *e = std::getenv("TCSEM_MARCH_PAIRS")) {

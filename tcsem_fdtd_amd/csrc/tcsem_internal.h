@@ -125,8 +125,8 @@ struct MarchArgs {
 // 2.  Step A stores its level 2 into the intermediate buffer (mex ..) and its running Bz sums
 // through level 2 into a.cs/a.cc; step B stores levels N-1 .. 3 and its sums through level 3 into
 // cs2/cc2.  The top levels of both steps are the ordinary top launches and surface kernels.
-// Tiles: 60 owned columns (64 lanes: two halo columns each side) by rows - 4 owned rows (two halo
-// rows each side); ntx, nty, nper count them (tiles per XCD group).
+// Tiles: pass_cols owned columns of 64 lanes (at least two halo columns each side) by rows - 4 owned rows (two
+// halo rows each side); ntx, nty, nper count them (tiles per XCD group).
 template <typename T>
 struct PairArgs {
   MarchArgs<T> a;                  // step A's scalars; old and new state; carry planes of step A
