@@ -238,6 +238,17 @@ long tcsem_graph_replays(const tcsem_ctx *ctx);
  * included), 0 when the march reads the full conductivity, -1 for no context. */
 int tcsem_sigma_table(const tcsem_ctx *ctx);
 
+/* The form of the air boundary that steps of nslot transmitters take (no counterpart in the reference,
+ * which has one): TCSEM_AIR_LINES, the line-by-line FFT chain (working lengths above 2048),
+ * TCSEM_AIR_FFT, the tiled FFT chain, or TCSEM_AIR_MATRIX, one real row operator per x wavenumber, built once
+ * per model.  TCSEM_UPCONT_CHAIN=lines, fft or dense in the environment at tcsem_create forces one.
+ * bytes (nullable): device memory that the context's row operators hold, 0 where there are none.
+ * Returns a negative code for no context or nslot < 1. */
+#define TCSEM_AIR_LINES 0
+#define TCSEM_AIR_FFT 1
+#define TCSEM_AIR_MATRIX 2
+int tcsem_air_form(const tcsem_ctx *ctx, int nslot, size_t *bytes);
+
 /* Two steps per lower pass (no counterpart in the reference, whose steps each read and write
  * the whole state): with rows 8, 10, 12, 14 or 16 (FP64: 8, 10, 11 or 12; workgroup rows of the pass) and pf 1 or 2 (prefetch
  * depth), tcsem_step and tcsem_run take each two consecutive steps after the source wavelet

@@ -116,6 +116,7 @@ def lib():
         "tcsem_set_graph": (C.c_int, [P, C.c_int]),
         "tcsem_graph_replays": (C.c_long, [P]),
         "tcsem_sigma_table": (C.c_int, [P]),
+        "tcsem_air_form": (C.c_int, [P, C.c_int, C.POINTER(C.c_size_t)]),
         "tcsem_set_pairs": (C.c_int, [P, C.c_int, C.c_int]),
         "tcsem_pair_info": (C.c_int, [P, ip, ip, C.POINTER(C.c_long)]),
         "tcsem_pair_timing": (C.c_int, [P, dp, C.POINTER(C.c_long)]),
@@ -397,6 +398,15 @@ class Context:
     def sigma_table(self):
         """Distinct conductivities (0 included) of the 8-bit index the march reads; 0: full values."""
         return self.L_.tcsem_sigma_table(self.h)
+
+    def air_form(self, nslot=1):
+        """(form of the air boundary for steps of nslot transmitters: "lines", "fft" or "matrix"; bytes of the
+        row operators that the context holds)."""
+        n = C.c_size_t()
+        f = self.L_.tcsem_air_form(self.h, nslot, C.byref(n))
+        if f < 0:
+            _check(f)
+        return ("lines", "fft", "matrix")[f], n.value
 
     def set_pairs(self, rows, pf=1):
         """Take two steps per lower pass (rows 8, 10, 12, 14 or 16 (FP64 8, 10, 11 or 12), prefetch pf 1 or 2; rows 0:

@@ -443,6 +443,7 @@ struct tcsem_ctx {
   // the air boundary in matrix form (choose_air): tables and row operators, one allocation
   int up_dense = 0;
   char *d_dn = nullptr;
+  size_t dn_bytes = 0;
   DenseOp dn{};
   double *d_scratch = nullptr;
   size_t scratch_bytes = 0;
@@ -2938,8 +2939,9 @@ int build_dense(tcsem_ctx *c) {
   const size_t nax = (size_t)(L + 15) / 16 * 16 * d.ldax, nb = (size_t)(2 * H + 3) / 4 * 4 * d.ldb;
   const size_t ntab = nax + 2 * nb + 2 * (size_t)(M / 2 + 1) + H;
   const size_t kb = (size_t)H * d.kstride * (d.kf32 ? 4 : 8);
-  if (hipMalloc(&c->d_dn, ntab * 8 + kb) != hipSuccess)
-    return fail(TCSEM_ENOMEM, "air operators: %zu bytes", ntab * 8 + kb);
+  c->dn_bytes = ntab * 8 + kb;
+  if (hipMalloc(&c->d_dn, c->dn_bytes) != hipSuccess)
+    return fail(TCSEM_ENOMEM, "air operators: %zu bytes", c->dn_bytes);
   double *p = (double *)c->d_dn;
   d.ax = b.ax = p;
   d.bx = b.bx = p + nax;
@@ -3063,7 +3065,7 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
     const char *chain = std::getenv("TCSEM_UPCONT_CHAIN");
     const bool want_lines = chain && std::strcmp(chain, "lines") == 0;
     c->up_tiled = !want_lines && c->plx.m <= 2048 && c->ply.m <= 2048 && L <= c->plx.m + 2 && M <= c->ply.m + 2;
-    c->up_dense = !want_lines && choose_air(c, chain);
+    c->up_dense = want_lines ? 0 : choose_air(c, chain);
     const bool chains = c->up_tiled || !c->up_dense;  // whether an FFT chain may run: its gains
     if (chains) {
       c->gx.assign((size_t)M1 * H, 0.0);
@@ -4091,6 +4093,14 @@ int tcsem_set_graph(tcsem_ctx *c, int nsteps) {
 }
 
 long tcsem_graph_replays(const tcsem_ctx *c) { return c ? c->graph_replays : -1; }
+
+int tcsem_air_form(const tcsem_ctx *c, int nslot, size_t *bytes) {
+  if (check_ctx(c)) return TCSEM_EINVAL;
+  if (nslot < 1) return fail(TCSEM_EINVAL, "at least one slot");
+  if (bytes) *bytes = c->d_dn ? c->dn_bytes : 0;
+  if (dense_pays(c->dn, c->prec == 32, nslot)) return TCSEM_AIR_MATRIX;
+  return c->up_tiled ? TCSEM_AIR_FFT : TCSEM_AIR_LINES;
+}
 
 int tcsem_sigma_table(const tcsem_ctx *c) { return c ? (c->s8 ? c->sig8_n : 0) : -1; }
 
