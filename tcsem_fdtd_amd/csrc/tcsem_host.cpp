@@ -2917,7 +2917,7 @@ int choose_air(tcsem_ctx *c, const char *chain) {
   d.w = (float)((1.8 * M * passes(c->plx) + 3.0 * (I.L1 / 2 + 1) * passes(c->ply)) * 1e-6);
   d.bm = (float)((double)I.L * M * I.N * 10.25 * c->esz * 1e-6);
   const bool f = c->prec == 32;
-  return dense_line(f, d.kb, d.w, d.bm) || dense_line(f, d.kb, 32 * d.w, 32 * d.bm) ? 1 : 0;
+  return dense_line(f, d.kb, d.w, d.bm) || dense_line(f, dense_reads(32) * d.kb, 32 * d.w, 32 * d.bm) ? 1 : 0;
 }
 
 // Builds the matrix form's operators on the device (c->dn, c->d_dn).

@@ -184,21 +184,27 @@ struct DenseOp {
   double *P, *Rx, *Ry;       // per slot 2 H x MP, slot stride sP
   long long sP;
 };
-// Whether the matrix form is faster than the tiled chain for a step of nslot slots.  It reads kb once per
-// step; the chain's time goes with its transforms' point passes w, but while the march takes longer
+// Slots that share one read of the row operators (k_dn_y's columns in LDS), and the reads of nslot slots.
+inline int dense_share(int nslot) { return nslot >= 4 ? 4 : nslot >= 2 ? 2 : 1; }
+inline int dense_reads(int nslot) { return (nslot + dense_share(nslot) - 1) / dense_share(nslot); }
+// Whether the matrix form is faster than the tiled chain for a step of nslot slots.  It reads its kb once per
+// dense_reads; the chain's time goes with its transforms' point passes w, but while the march takes longer
 // than the chain (bm: the march's bytes) the chain hides beside it and the operators' bytes do not.  The
-// line between was fitted to whole runs, us per step chain / matrix form (kb, w, bm for one slot):
-//   FP32 100 x 100 x 60 under 356 x 356 (7, 15, 25) 87 / 57; 320 x 320 x 60 under 576 x 576 (119, 65, 252)
-//     149 / 126; 320 x 320 x 160 (119, 65, 672) 224 / 245; 420 x 400 x 60 under 676 x 656 (217, 78, 413) 183 / 216;
-//     256 x 256 x 60 under 512 x 512 (68, 6, 161) 93 / 94; 200 x 200 x 160 under 712 x 712 (57, 65, 262) 167 / 131;
-//     300 x 300 x 60 under 556 x 556, 2 slots 217 / 192, 8 slots 761 / 544;
-//   FP64 100 x 100 x 60 103 / 68; 320 x 320 x 60 (238, 65, 504) 252 / 227; 420 x 400 x 60 (435, 78, 827) 342 / 362;
-//     360 x 350 x 160 under 616 x 606 (304, 70, 1653) 512 / 534; 300 x 300 x 60, 2 slots 402 / 325, 8 slots 1749 / 837.
+// line between was fitted to whole runs one step at a time; us per step of today's runs, chain / matrix form (kb, w, bm
+// for one slot), in pairs but for the grids of 100 x 100:
+//   FP32 100 x 100 x 60 under 356 x 356 (7, 15, 25) 85 / 56; 320 x 320 x 60 under 576 x 576 (119, 65, 252)
+//     128 / 106; 320 x 320 x 160 (119, 65, 672) 168 / 167; 420 x 400 x 60 under 676 x 656 (217, 78, 413) 152 / 179;
+//     256 x 256 x 60 under 512 x 512 (68, 6, 161) 73.1 / 73.2; 200 x 200 x 160 under 712 x 712 (57, 65, 262) 141 / 112;
+//     300 x 300 x 60 under 556 x 556, 2 slots 173 / 157, 8 slots 664 / 480, 32 slots 2464 / 1863;
+//   FP64 100 x 100 x 60 101 / 67; 320 x 320 x 60 (238, 65, 504) 214 / 173; 420 x 400 x 60 (435, 78, 827) 255 / 267;
+//     360 x 350 x 160 under 616 x 606 (304, 70, 1653) 348 / 341; 300 x 300 x 60, 2 slots 335 / 218, 16 slots 3001 / 1363;
+//   many slots of shallow grids under powers of two, whose transforms are cheap: FP32 512 x 512 x 10 under 1024 x 1024,
+//     16 slots (539, 25, 107) 937 / 2094; 256 x 256 x 12, 32 slots (68, 6, 32) 550 / 778; FP64, 16 slots 418 / 503.
 inline bool dense_line(bool fp32, float kb, float w, float bm) {
   return fp32 ? 4.75f * w - 0.46f * bm + 30.f > kb : 6.75f * w - 0.175f * bm + 30.f > kb;
 }
 inline bool dense_pays(const DenseOp &d, bool fp32, int nslot) {
-  return d.on == 2 || (d.on == 1 && dense_line(fp32, d.kb, d.w * nslot, d.bm * nslot));
+  return d.on == 2 || (d.on == 1 && dense_line(fp32, d.kb * dense_reads(nslot), d.w * nslot, d.bm * nslot));
 }
 // Building them: the tables above, cosine/sine tables per ky (pitch ldy) and the folded gains.
 struct DenseBuild {

@@ -14,9 +14,9 @@
 // Built once per model on the device; FP64 data and sums throughout (the row operators are kept in
 // FP32 where the FFT chain that they replace computes in FP32: their sums are FP64 here).
 //
-// Bound: k_dn_y reads every operator entry once per call (2 M (M + 1/2) H words), which the FFT chain
-// replaces by transforms: it wins where those are long against the irregular rows or not powers of
-// two (the rule is in the host's choose_air).  The two products run at a fraction of the FP64 matrix rate
+// Bound: k_dn_y reads every operator entry once per four slots (M (M + 1/2) H words), which the FFT chain
+// replaces by transforms: the matrix form wins where those are long against the irregular rows or not powers of
+// two (the rule is dense_pays).  The two products run at a fraction of the FP64 matrix rate
 // (6 M L L1 flops).
 #include "tcsem_internal.h"
 
@@ -235,8 +235,9 @@ hipError_t launch_dn_y(const UpcontArgs<T> &u, int nslot, hipStream_t s, const U
 template <typename T, typename TK, bool GEO>
 hipError_t launch_dn_y_ns(const UpcontArgs<T> &u, int nslot, hipStream_t s, const UpcontArgs<T> *geo) {
   if constexpr (!GEO) {
-    if (nslot >= 4) return launch_dn_y<T, TK, 4, GEO>(u, nslot, s, geo);
-    if (nslot >= 2) return launch_dn_y<T, TK, 2, GEO>(u, nslot, s, geo);
+    const int ns = dense_share(nslot);
+    if (ns == 4) return launch_dn_y<T, TK, 4, GEO>(u, nslot, s, geo);
+    if (ns == 2) return launch_dn_y<T, TK, 2, GEO>(u, nslot, s, geo);
   }
   return launch_dn_y<T, TK, 1, GEO>(u, nslot, s, geo);
 }

@@ -69,6 +69,18 @@ def test_own_choice(kw, form):
         assert f == form and (n > 0) == (form == "matrix")
 
 
+@pytest.mark.parametrize("precision", [T.FP32, T.FP64])
+def test_own_choice_of_many_slots(precision):
+    """Four slots share a read of the row operators: 32 slots of a shallow grid under 512 x 512 regular points read
+    them eight times, which costs more than the transforms (778 us a step against 550 in FP32)."""
+    st = decks.small_setup(T, nx=216, ny=216, nz=12, pad=(6, 14), arg=(1.05, 1.747))
+    st.Az1 = st.Az2 = 0
+    gi = T.grid_info(st)
+    assert (gi.L, gi.M, gi.N, gi.L1, gi.M1) == (256, 256, 12, 512, 512)
+    with T.Context(st, np.ones((gi.N, gi.M, gi.L)), precision) as c:
+        assert [c.air_form(n)[0] for n in (16, 32)] == ["fft"] * 2
+
+
 TXS = [dict(B.TX, x=x, txid=q + 1) for q, x in enumerate((0.0, -100.0, 120.0, 60.0))]
 COND = B.CONDS[0]
 _REF = {}
