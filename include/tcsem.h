@@ -301,6 +301,10 @@ int tcsem_batch_timing(tcsem_batch *batch, double t[3], long n[3]);
  * of the last step call (0: one step at a time), the autotuner's pick (-1: not tuned) and the
  * pairs taken; tcsem_batch_pair_timing: the pass's average device time while timing is enabled. */
 int tcsem_batch_set_pairs(tcsem_batch *batch, int rows);
+/* Form of the air boundary, one for every member (TCSEM_AIR_FFT or TCSEM_AIR_MATRIX), chosen at tcsem_batch_create
+ * from the members' sizes together; row operators that members lack for it are built there.  A member run
+ * alone may take the other form: its traces agree to round-off then. */
+int tcsem_batch_air_form(const tcsem_batch *batch);
 int tcsem_batch_pair_info(const tcsem_batch *batch, int *rows, int *tuned, long *pairs);
 int tcsem_batch_pair_timing(tcsem_batch *batch, double *ms, long *n);
 void tcsem_batch_destroy(tcsem_batch *batch);

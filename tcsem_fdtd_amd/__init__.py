@@ -128,6 +128,7 @@ def lib():
         "tcsem_batch_destroy": (None, [P]),
         "tcsem_batch_enable_timing": (C.c_int, [P, C.c_int]),
         "tcsem_batch_timing": (C.c_int, [P, dp, C.POINTER(C.c_long)]),
+        "tcsem_batch_air_form": (C.c_int, [P]),
         "tcsem_batch_set_pairs": (C.c_int, [P, C.c_int]),
         "tcsem_batch_pair_info": (C.c_int, [P, ip, ip, C.POINTER(C.c_long)]),
         "tcsem_batch_pair_timing": (C.c_int, [P, dp, C.POINTER(C.c_long)]),
@@ -461,6 +462,13 @@ class Batch:
         r, p, ms = C.c_int(), C.c_int(), C.c_double()
         _check(self.L_.tcsem_batch_autotune(self.h, nsteps, C.byref(r), C.byref(p), C.byref(ms)))
         return {"rows": r.value, "pf": p.value, "pairs": self.pair_info()[1] or None, "step_ms": ms.value}
+
+    def air_form(self):
+        """Form of the members' air boundary: "fft" or "matrix"."""
+        f = self.L_.tcsem_batch_air_form(self.h)
+        if f < 0:
+            _check(f)
+        return ("lines", "fft", "matrix")[f]
 
     def set_pairs(self, rows):
         """Two steps per pass for the batch (rows 8, 10, 12, 14 or 16, FP64 8, 10, 11 or 12; 0: one at a time)."""

@@ -438,9 +438,11 @@ struct tcsem_ctx {
   // upward-continuation work: the tiled chain's A, G, bxr, byr regions (slot strides sA, sG, sX
   // doubles), or the line chain's cplx (complex), tx, bxr, byr regions (wstride each)
   double *d_work = nullptr;
+  size_t work_cap = 0;
   int up_tiled = 0, MA = 0, MG = 0, XR = 0;
   long long sA = 0, sG = 0, sX = 0;
-  // the air boundary in matrix form (choose_air): tables and row operators, one allocation
+  // the air boundary in matrix form: whether it may be taken (0 no, 1 by dense_pays, 2 always), and its tables and
+  // row operators, one allocation (null: not built)
   int up_dense = 0;
   char *d_dn = nullptr;
   size_t dn_bytes = 0;
@@ -817,7 +819,7 @@ UpcontArgs<T> upcont_args(tcsem_ctx *c) {
   double *w = c->d_work;
   u.tiled = c->up_tiled;
   u.d = c->dn;
-  if (c->up_dense) {  // the matrix form's planes share the work buffer with the chain's
+  if (c->d_dn) {  // the matrix form's planes share the work buffer with the chain's
     const long long ns = c->nslots;
     u.d.P = w;
     u.d.Rx = w + ns * c->dn.sP;
@@ -893,8 +895,28 @@ void free_run(tcsem_ctx *c) {
   c->begun = false;
 }
 
+// Work planes of the air boundary for c->nslots slots.  Bytes per slot: tiled chain A and G (complex of the field
+// type) and Bx, By (field type); line chain cplx (complex FP64), tx, bxr (also the y-padding rows), byr (FP64); the
+// matrix form 3 planes of 2 H x MP (FP64), beside the tiled chain's need (the slot count decides between them), in
+// place of the line chain's.  Called again after the operators were built: the planes may grow.
+int reserve_work(tcsem_ctx *c) {
+  const size_t chain = c->up_tiled ? (size_t)(2 * c->sA + 2 * c->sG + 2 * c->sX) * c->esz
+                                   : (c->up_dense ? 0 : (size_t)5 * c->wstride * sizeof(double));
+  const size_t wb = (size_t)c->nslots * std::max(chain, (size_t)(3 * c->dn.sP) * sizeof(double));
+  if (wb <= c->work_cap) return TCSEM_OK;
+  drop_graphs(c);
+  HIPCHK(hipStreamSynchronize(c->stream2));
+  HIPCHK(hipStreamSynchronize(c->stream));
+  (void)hipFree(c->d_work);
+  c->d_work = nullptr;
+  c->work_cap = 0;
+  if (hipMalloc((void **)&c->d_work, wb) != hipSuccess) return fail(TCSEM_ENOMEM, "work allocation failed");
+  c->work_cap = wb;
+  return TCSEM_OK;
+}
+
 int alloc_slots(tcsem_ctx *c, int nslots) {
-  if (nslots <= c->nslots) return TCSEM_OK;
+  if (nslots <= c->nslots) return reserve_work(c);
   drop_graphs(c);
   HIPCHK(hipStreamSynchronize(c->stream));
   (void)hipFree(c->d_fields);
@@ -909,20 +931,12 @@ int alloc_slots(tcsem_ctx *c, int nslots) {
   c->ib_valid = false;
   c->d_fields = c->d_planes = c->d_zs = nullptr;
   c->d_work = nullptr;
+  c->work_cap = 0;
   c->nslots = 0;
   const size_t fb = (size_t)2 * 5 * nslots * c->fstride * c->esz;
   const size_t pb = (size_t)7 * nslots * c->pstride * c->esz;
-  // bytes per slot: tiled chain A and G (complex of the field type) and Bx, By (field type);
-  // line chain cplx (complex FP64), tx, bxr (also the y-padding rows), byr (FP64)
-  // the matrix form 3 planes of 2 H x MP (FP64), beside the tiled chain's need (a model batch may run
-  // either), in place of the line chain's
-  const size_t chain = c->up_tiled ? (size_t)(2 * c->sA + 2 * c->sG + 2 * c->sX) * c->esz
-                                   : (c->up_dense ? 0 : (size_t)5 * c->wstride * sizeof(double));
-  const size_t per_slot = std::max(chain, (size_t)(3 * c->dn.sP) * sizeof(double));
-  const size_t wb = (size_t)nslots * per_slot;
   if (hipMalloc(&c->d_fields, fb) != hipSuccess) return fail(TCSEM_ENOMEM, "field allocation of %zu bytes failed", fb);
   if (hipMalloc(&c->d_planes, pb) != hipSuccess) return fail(TCSEM_ENOMEM, "plane allocation failed");
-  if (hipMalloc((void **)&c->d_work, wb) != hipSuccess) return fail(TCSEM_ENOMEM, "work allocation failed");
   const size_t zb = (size_t)(kMaxChunks - 1) * nslots * c->pstride * c->esz;
   if (hipMalloc(&c->d_zs, zb) != hipSuccess) return fail(TCSEM_ENOMEM, "chunk-sum allocation failed");
   HIPCHK(launch_fill_zero(c->d_zs, zb, c->stream));
@@ -931,6 +945,10 @@ int alloc_slots(tcsem_ctx *c, int nslots) {
   HIPCHK(hipStreamSynchronize(c->stream));
   c->nslots = nslots;
   c->cur = 0;
+  if (const int rc = reserve_work(c)) {
+    c->nslots = 0;
+    return rc;
+  }
   return TCSEM_OK;
 }
 
@@ -2021,6 +2039,7 @@ struct tcsem_batch {
   size_t pwork_cap = 0;
   int pwork_len = 0;
   long pairs_done = 0;
+  bool air_mat = false;  // the air boundary of every member in matrix form (batch_air)
 };
 
 namespace {
@@ -2162,20 +2181,8 @@ int batch_records(tcsem_batch *b, int by, int pf, MarchArgs<T> &la, UpcontArgs<T
   la.k_hi = la.N - 1;
   la.k_lo = 1;
   ul.tiled = 1;
-  // the matrix form of the air boundary when every member has it (of one kind), else the tiled chain for all
-  {
-    ul.d = b->m[0]->dn;
-    bool have = true, always = false;
-    float kb = 0, w = 0, bm = 0;
-    for (const tcsem_ctx *c : b->m) {
-      have = have && c->dn.on && c->dn.kf32 == ul.d.kf32;
-      always = always || c->dn.on == 2;
-      kb += c->dn.kb;
-      w += c->dn.w;
-      bm += c->dn.bm;
-    }
-    ul.d.on = have && (always || dense_line(b->prec == 32, kb, w, bm)) ? 2 : 0;
-  }
+  ul.d = b->m[0]->dn;
+  ul.d.on = b->air_mat ? 2 : 0;
   // the march's work list
   {
     std::vector<int> tiles(nm);
@@ -2886,10 +2893,10 @@ int tcsem_waveform(int ns, double sigma_t, double *t, double *dt, double *wave) 
 
 extern "C++" {
 namespace {
-// Whether the matrix form of the air boundary is built (chain: TCSEM_UPCONT_CHAIN; "dense" and "fft" force it
+// Whether the matrix form of the air boundary may be taken (chain: TCSEM_UPCONT_CHAIN; "dense" and "fft" force it
 // on and off): 2 where it always runs -- beyond the tiled chain (working lengths over 2048) the line chain is
-// slower by an order of magnitude: 220 x 200 x 110 under 3914 x 3894, FP64, 60 steps: 481.8 ms / 22.3 ms --,
-// 1 where it runs for some number of slots (dense_pays).
+// slower by an order of magnitude: 220 x 200 x 110 under 3914 x 3894, FP64, 60 steps: 481.8 ms / 17.1 ms --,
+// 1 where it runs for the slot counts of dense_pays; sets what that goes by.
 constexpr size_t kDenseMax = (size_t)16 << 30;  // row operators of one model
 int choose_air(tcsem_ctx *c, const char *chain) {
   const HostGrid &g = c->g;
@@ -2908,7 +2915,7 @@ int choose_air(tcsem_ctx *c, const char *chain) {
   // the allocation-free entry point's work planes have to hold it where the tiled chain's fit them; LDS of
   // k_dn_y at four slots
   if (bytes > kDenseMax || (c->up_tiled && work > kUpcontScratchBytes) || M > 800) return 0;
-  if (!c->up_tiled || (chain && std::strcmp(chain, "dense") == 0)) return 2;
+  if (!c->up_tiled) return 2;
   // point passes of the tiled chain: rows in and out along x, three transforms of each column, two working
   // lengths each where Bluestein's
   auto passes = [](const HostPlan &p) { return (p.m == p.n ? 1.0 : 2.0) * p.m * p.log2m; };
@@ -2916,8 +2923,14 @@ int choose_air(tcsem_ctx *c, const char *chain) {
   d.kb = (float)(bytes * 1e-6);
   d.w = (float)((1.8 * M * passes(c->plx) + 3.0 * (I.L1 / 2 + 1) * passes(c->ply)) * 1e-6);
   d.bm = (float)((double)I.L * M * I.N * 10.25 * c->esz * 1e-6);
-  const bool f = c->prec == 32;
-  return dense_line(f, d.kb, d.w, d.bm) || dense_line(f, dense_reads(32) * d.kb, 32 * d.w, 32 * d.bm) ? 1 : 0;
+  return chain && std::strcmp(chain, "dense") == 0 ? 2 : 1;
+}
+
+// Whether a step of nslot slots takes the matrix form once its operators are built.
+bool wants_dense(const tcsem_ctx *c, int nslot) {
+  DenseOp d = c->dn;
+  d.on = c->up_dense;
+  return dense_pays(d, c->prec == 32, nslot);
 }
 
 // Builds the matrix form's operators on the device (c->dn, c->d_dn).
@@ -2926,7 +2939,6 @@ int build_dense(tcsem_ctx *c) {
   const int L = I.L, M = I.M, L1 = I.L1, M1 = I.M1, H = L1 / 2 + 1;
   DenseOp &d = c->dn;
   DenseBuild b{};
-  d.on = c->up_dense;
   d.kf32 = c->up_tiled && c->prec == 32;
   d.ldax = b.ldax = (2 * H + 31) / 32 * 32;
   d.ldb = b.ldb = (L + 1 + 15) / 16 * 16;
@@ -2969,7 +2981,13 @@ int build_dense(tcsem_ctx *c) {
   }
   const size_t ny = (size_t)b.Hy * b.ldy, ng = (size_t)H * b.Hy, ntmp = trig.size() + 6 * ny + 2 * ng;
   double *t = nullptr;
-  if (hipMalloc((void **)&t, ntmp * 8) != hipSuccess) return fail(TCSEM_ENOMEM, "air operator tables: %zu bytes", ntmp * 8);
+  auto drop = [&](int code) {
+    (void)hipFree(c->d_dn);
+    c->d_dn = nullptr;
+    return code;
+  };
+  if (hipMalloc((void **)&t, ntmp * 8) != hipSuccess)
+    return drop(fail(TCSEM_ENOMEM, "air operator tables: %zu bytes", ntmp * 8));
   b.tx = (const double2 *)t;
   b.ty = b.tx + L1;
   b.cw = t + trig.size();
@@ -2986,7 +3004,40 @@ int build_dense(tcsem_ctx *c) {
   if (e == hipSuccess) e = launch_dense_build(b, upcont_args<double>(c), d.kf32 != 0, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   (void)hipFree(t);
-  if (e != hipSuccess) return fail(TCSEM_EDEVICE, "air operators: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return drop(fail(TCSEM_EDEVICE, "air operators: %s", hipGetErrorString(e)));
+  d.on = c->up_dense;
+  return TCSEM_OK;
+}
+
+// Builds the operators of a context in use, where it has none.
+int ensure_dense(tcsem_ctx *c) {
+  if (c->d_dn) return TCSEM_OK;
+  int rc = build_dense(c);
+  if (!rc) rc = reserve_work(c);
+  if (rc) return rc;
+  c->up64 = upcont_args<double>(c);
+  c->up32 = upcont_args<float>(c);
+  return TCSEM_OK;
+}
+
+// The form of a batch's air boundary, one for all members: two sets of launches, each member in the form that it takes
+// alone, cost more than either (64 uneven models FP32, all but six in matrix form, ms a step: chain 2.21,
+// matrix form 2.19, mixed 2.27; one member on the chain of two FP64 0.148, mixed 0.182).  The members' sizes add up
+// in the rule; operators that a member lacks are built here.
+int batch_air(tcsem_batch *b) {
+  bool may = true, always = false;
+  float kb = 0, w = 0, bm = 0;
+  for (const tcsem_ctx *c : b->m) {
+    may = may && c->up_dense;
+    always = always || c->up_dense == 2;
+    kb += c->dn.kb;
+    w += c->dn.w;
+    bm += c->dn.bm;
+  }
+  if (!may || !(always || dense_line(b->prec == 32, kb, w, bm))) return TCSEM_OK;
+  for (tcsem_ctx *c : b->m)
+    if (int rc = ensure_dense(c)) return rc;
+  b->air_mat = true;
   return TCSEM_OK;
 }
 }  // namespace
@@ -3283,7 +3334,7 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
     if (hipMemcpy(c->d_up, up.data(), up.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(TCSEM_EDEVICE, "operator upload"));
   }
-  if (c->up_dense && (rc = build_dense(c))) return bail(rc);
+  if ((wants_dense(c, 1) || wants_dense(c, 32)) && (rc = build_dense(c))) return bail(rc);
   if ((rc = alloc_slots(c, 1))) return bail(rc);
   c->nbatch = 1;
   c->up64 = upcont_args<double>(c);
@@ -4004,6 +4055,10 @@ int tcsem_batch_create(tcsem_ctx *const *models, int nmodel, tcsem_batch **out) 
     tcsem_batch_destroy(b);
     return fail(TCSEM_EDEVICE, "batch stream, event or record allocation failed");
   }
+  if (const int rc = batch_air(b)) {
+    tcsem_batch_destroy(b);
+    return rc;
+  }
   *out = b;
   return TCSEM_OK;
 }
@@ -4100,6 +4155,11 @@ int tcsem_air_form(const tcsem_ctx *c, int nslot, size_t *bytes) {
   if (bytes) *bytes = c->d_dn ? c->dn_bytes : 0;
   if (dense_pays(c->dn, c->prec == 32, nslot)) return TCSEM_AIR_MATRIX;
   return c->up_tiled ? TCSEM_AIR_FFT : TCSEM_AIR_LINES;
+}
+
+int tcsem_batch_air_form(const tcsem_batch *b) {
+  if (!b) return fail(TCSEM_EINVAL, "null batch");
+  return b->air_mat ? TCSEM_AIR_MATRIX : TCSEM_AIR_FFT;
 }
 
 int tcsem_sigma_table(const tcsem_ctx *c) { return c ? (c->s8 ? c->sig8_n : 0) : -1; }

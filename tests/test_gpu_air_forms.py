@@ -169,3 +169,63 @@ def test_batch(chain, precision, tol, rows, monkeypatch):
     finally:
         for c in cx:
             c.close()
+
+
+def _marine(n, nz):
+    """A grid of n x n x nz cells under n + 256 regular points a side."""
+    st = decks.small_setup(T, nx=n - 40, ny=n - 40, nz=nz, pad=(6, 14), arg=(1.05, 1.747))
+    st.Az1 = st.Az2 = 0
+    return st
+
+
+@pytest.mark.parametrize("precision,tol", [(T.FP64, 1e-11), (T.FP32, 1e-5)])
+@pytest.mark.parametrize("rows", [0, 8])
+@pytest.mark.parametrize("sides,form", [((256, 100, 100), "matrix"), ((256, 256, 100), "fft")])
+def test_batch_form(sides, form, precision, tol, rows):
+    """The batch's members together decide: a 256 x 256 grid alone stays with the chain, and two of 100 x 100 carry it
+    over to row operators built for the batch, unless a second one of 256 x 256 comes with it.  Each member equals its
+    run alone to round-off."""
+    cx = []
+    try:
+        for q, n in enumerate(sides):
+            st = _marine(n, 24)
+            gi = T.grid_info(st)
+            cond = decks.layered_cond((gi.N, gi.M, gi.L), T.grid_arrays(st)["Z"][:, None, None] *
+                                      np.ones((1, gi.M, gi.L)), seed=q)
+            c = T.Context(st, cond, precision)
+            c.set_receivers(B._rt(T, 0.08 if q == 1 else 0.25), B.RX)
+            c.set_transmitters([T.make_tx(**B.TX)])
+            c.set_pairs(8)
+            c.set_graph(0)
+            cx.append(c)
+            assert c.air_form()[0] == ("fft" if n == 256 else "matrix")
+        alone = [c.run(0, 1, max_steps=300)[0] for c in cx]
+        with T.Batch(cx) as b:
+            b.set_pairs(rows)
+            b.enable_timing()
+            assert b.air_form() == form
+            got = b.run(max_steps=300)
+            assert b.timing()["upcont_ms"] > 0.0
+        for c, n, a, g in zip(cx, sides, alone, got):
+            assert np.any(a != 0)
+            assert np.all(decks.trace_error(g, a) < tol)
+        again = [c.run(0, 1, max_steps=300)[0] for c in cx]  # a member keeps its own form, operators or not
+        for a, g in zip(alone, again):
+            assert np.array_equal(a, g)
+    finally:
+        for c in cx:
+            c.close()
+
+
+def test_batch_of_a_member_without_the_matrix_form(monkeypatch):
+    cx = []
+    try:
+        for kw, cond, chain in zip(B.MODELS, B.CONDS, ("dense", "fft")):
+            monkeypatch.setenv("TCSEM_UPCONT_CHAIN", chain)
+            cx.append(B._ctx(kw, cond, T.FP64))
+        with T.Batch(cx) as b:
+            assert b.air_form() == "fft"
+            b.run(max_steps=60)
+    finally:
+        for c in cx:
+            c.close()
