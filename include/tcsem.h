@@ -241,7 +241,8 @@ int tcsem_sigma_table(const tcsem_ctx *ctx);
 /* The form of the air boundary that steps of nslot transmitters take (no counterpart in the reference,
  * which has one): TCSEM_AIR_LINES, the line-by-line FFT chain (working lengths above 2048),
  * TCSEM_AIR_FFT, the tiled FFT chain, or TCSEM_AIR_MATRIX, one real row operator per x wavenumber, built once
- * per model.  TCSEM_UPCONT_CHAIN=lines, fft or dense in the environment at tcsem_create forces one.
+ * per model, at tcsem_create where steps of one transmitter take them, else at the first tcsem_reserve_batch, tcsem_begin or
+ * tcsem_batch_create that calls for them.  TCSEM_UPCONT_CHAIN=lines, fft or dense in the environment at tcsem_create forces one.
  * bytes (nullable): device memory that the context's row operators hold, 0 where there are none.
  * Returns a negative code for no context or nslot < 1. */
 #define TCSEM_AIR_LINES 0

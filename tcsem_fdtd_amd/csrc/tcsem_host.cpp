@@ -3334,7 +3334,8 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
     if (hipMemcpy(c->d_up, up.data(), up.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(TCSEM_EDEVICE, "operator upload"));
   }
-  if ((wants_dense(c, 1) || wants_dense(c, 32)) && (rc = build_dense(c))) return bail(rc);
+  // one slot: what the plane calls need, which may allocate nothing; more where they are reserved
+  if (wants_dense(c, 1) && (rc = build_dense(c))) return bail(rc);
   if ((rc = alloc_slots(c, 1))) return bail(rc);
   c->nbatch = 1;
   c->up64 = upcont_args<double>(c);
@@ -3473,8 +3474,9 @@ int tcsem_set_transmitters(tcsem_ctx *c, const tcsem_tx *tx, int ntx) {
 
 int tcsem_reserve_batch(tcsem_ctx *c, int nbatch) {
   if (check_ctx(c) || nbatch < 1) return fail(TCSEM_EINVAL, "bad batch size");
-  const int rc = alloc_slots(c, nbatch);
-  if (rc) return rc;
+  int rc = TCSEM_OK;
+  if (!c->d_dn && wants_dense(c, nbatch) && (rc = build_dense(c))) return rc;
+  if ((rc = alloc_slots(c, nbatch))) return rc;
   c->up64 = upcont_args<double>(c);
   c->up32 = upcont_args<float>(c);
   return TCSEM_OK;
@@ -4153,7 +4155,7 @@ int tcsem_air_form(const tcsem_ctx *c, int nslot, size_t *bytes) {
   if (check_ctx(c)) return TCSEM_EINVAL;
   if (nslot < 1) return fail(TCSEM_EINVAL, "at least one slot");
   if (bytes) *bytes = c->d_dn ? c->dn_bytes : 0;
-  if (dense_pays(c->dn, c->prec == 32, nslot)) return TCSEM_AIR_MATRIX;
+  if (wants_dense(c, nslot)) return TCSEM_AIR_MATRIX;
   return c->up_tiled ? TCSEM_AIR_FFT : TCSEM_AIR_LINES;
 }
 

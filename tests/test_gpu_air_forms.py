@@ -81,6 +81,41 @@ def test_own_choice_of_many_slots(precision):
         assert [c.air_form(n)[0] for n in (16, 32)] == ["fft"] * 2
 
 
+def test_operators_are_built_where_they_are_used(monkeypatch):
+    """420 x 400 x 64 FP32: one transmitter stays with the chain, eight take the matrix form.  A context that never runs
+    eight holds no operators, one that does runs them as a context that had them from the start, and its one-slot calls
+    stay as they were."""
+    st = decks.small_setup(T, nx=380, ny=360, nz=64, pad=(6, 14), arg=(1.05, 1.747))
+    st.Az1 = st.Az2 = 0
+    gi = T.grid_info(st)
+    assert (gi.L, gi.M, gi.N) == (420, 400, 64)
+    cond = np.ones((gi.N, gi.M, gi.L))
+    bz0 = np.random.default_rng(5).standard_normal((gi.M, gi.L))
+    txs = [T.make_tx(1, 100.0, 200.0 * q - 700.0, 0.0, 100.0, [1]) for q in range(8)]
+    out = []
+    for chain in ("", "dense"):
+        monkeypatch.setenv("TCSEM_UPCONT_CHAIN", chain)
+        with T.Context(st, cond, T.FP32) as c:
+            c.set_receivers(B._rt(T), np.array([[0.0, 100.0, 400.0]]))
+            c.set_transmitters(txs)
+            if not chain:
+                assert c.air_form(1) == ("fft", 0) and c.air_form(8)[0] == "matrix"
+                plane = c.upcont_plane(bz0)
+                c.begin(0, 1)
+                assert c.air_form(1) == ("fft", 0)
+            c.begin(0, 8)
+            f, n = c.air_form(8)
+            assert f == "matrix" and n > 2e8
+            c.step(8)
+            out.append([c.get(T.BXAIR, q) for q in range(8)])
+            if not chain:
+                assert c.air_form(1)[0] == "fft"
+                for a, b in zip(plane, c.upcont_plane(bz0)):
+                    assert np.array_equal(a, b)
+    for a, b in zip(*out):
+        assert np.any(a) and np.array_equal(a, b)
+
+
 TXS = [dict(B.TX, x=x, txid=q + 1) for q, x in enumerate((0.0, -100.0, 120.0, 60.0))]
 COND = B.CONDS[0]
 _REF = {}
