@@ -243,7 +243,8 @@ int tcsem_sigma_table(const tcsem_ctx *ctx);
  * TCSEM_AIR_FFT, the tiled FFT chain, or TCSEM_AIR_MATRIX, one real row operator per x wavenumber, built once
  * per model, at tcsem_create where steps of one transmitter take them, else at the first tcsem_reserve_batch, tcsem_begin or
  * tcsem_batch_create that calls for them.  TCSEM_UPCONT_CHAIN=lines, fft or dense in the environment at tcsem_create forces one.
- * bytes (nullable): device memory that the context's row operators hold, 0 where there are none.
+ * TCSEM_SPARE_MB in the environment keeps that much device memory free of them; a context without room for them runs its
+ * FFT chain.  bytes (nullable): device memory that the context's row operators hold, 0 where there are none.
  * Returns a negative code for no context or nslot < 1. */
 #define TCSEM_AIR_LINES 0
 #define TCSEM_AIR_FFT 1

@@ -445,6 +445,7 @@ struct tcsem_ctx {
   // row operators, one allocation (null: not built)
   int up_dense = 0;
   char *d_dn = nullptr;
+  double *d_dnt = nullptr;  // tables that the operators are built from (freed once they are)
   size_t dn_bytes = 0;
   DenseOp dn{};
   double *d_scratch = nullptr;
@@ -863,6 +864,21 @@ UpcontArgs<T> upcont_args(tcsem_ctx *c) {
   u.yrows = u.yBy2N + I.M + 1;
   u.nyr = c->nyr;
   return u;
+}
+
+// Device memory that a run can do without: refused, with no error left behind, where it does not fit, where it would
+// take more than 1/share of the free memory, or where it would not leave TCSEM_SPARE_MB free.
+hipError_t optional_malloc(void **p, size_t bytes, size_t share) {
+  *p = nullptr;
+  const char *e = std::getenv("TCSEM_SPARE_MB");
+  const double spare = e ? std::atof(e) * 1e6 : 0.0;
+  size_t avail = 0, total = 0;
+  if (hipMemGetInfo(&avail, &total) == hipSuccess && (double)bytes * share <= (double)avail - spare &&
+      hipMalloc(p, bytes) == hipSuccess)
+    return hipSuccess;
+  (void)hipGetLastError();
+  *p = nullptr;
+  return hipErrorOutOfMemory;
 }
 
 // Graph executables bake device addresses: dropped whenever an allocation they use may change.
@@ -2933,44 +2949,81 @@ bool wants_dense(const tcsem_ctx *c, int nslot) {
   return dense_pays(d, c->prec == 32, nslot);
 }
 
-// Builds the matrix form's operators on the device (c->dn, c->d_dn).
+// Sizes of the operators and of the tables that they are built from, in doubles but for kb (bytes).
+struct DenseSizes {
+  int ldax, ldb, MP, Hy, ldy;
+  long long kstride;
+  size_t nax, nb, ntab, kb, ntrig, ny, ng;
+};
+DenseSizes dense_sizes(const tcsem_ctx *c, bool kf32) {
+  const tcsem_grid_info &I = c->g.info;
+  const int L = I.L, M = I.M, H = I.L1 / 2 + 1, ne = (M + 1) / 2, no = M / 2;
+  DenseSizes z;
+  z.ldax = (2 * H + 31) / 32 * 32;
+  z.ldb = (L + 1 + 15) / 16 * 16;
+  z.MP = (M + 1 + 31) / 32 * 32;
+  z.Hy = I.M1 / 2 + 1;
+  z.ldy = (M / 2 + 1 + 31) / 32 * 32;
+  z.kstride = (long long)ne * (ne + (M + 1) / 2) + (long long)no * (no + M / 2 + 1);
+  z.nax = (size_t)(L + 15) / 16 * 16 * z.ldax;
+  z.nb = (size_t)(2 * H + 3) / 4 * 4 * z.ldb;
+  z.ntab = z.nax + 2 * z.nb + 2 * (size_t)(M / 2 + 1) + H;
+  z.kb = (size_t)H * z.kstride * (kf32 ? 4 : 8);
+  z.ntrig = 2 * (size_t)I.L1 + 4 * (size_t)I.M1;
+  z.ny = (size_t)z.Hy * z.ldy;
+  z.ng = (size_t)H * z.Hy;
+  return z;
+}
+
+// Their device memory; false, and the context stays with its FFT chain, where there is no room.  Beside the tiled chain
+// they may take a sixteenth of what is free; beyond it the line chain is so much slower, and needs as much itself,
+// that they may take all.
+bool alloc_dense(tcsem_ctx *c) {
+  const DenseSizes z = dense_sizes(c, c->up_tiled && c->prec == 32);
+  const size_t share = c->up_tiled ? 16 : 1;
+  c->dn_bytes = z.ntab * 8 + z.kb;
+  if (optional_malloc((void **)&c->d_dn, c->dn_bytes, share) == hipSuccess &&
+      optional_malloc((void **)&c->d_dnt, (z.ntrig + 6 * z.ny + 2 * z.ng) * 8, share) == hipSuccess)
+    return true;
+  (void)hipFree(c->d_dn);
+  c->d_dn = nullptr;
+  c->up_dense = 0;
+  return false;
+}
+
+// Builds the matrix form's operators on the device (c->dn, c->d_dn) where there is room for them.
 int build_dense(tcsem_ctx *c) {
   const tcsem_grid_info &I = c->g.info;
-  const int L = I.L, M = I.M, L1 = I.L1, M1 = I.M1, H = L1 / 2 + 1;
+  const int M = I.M, L1 = I.L1, M1 = I.M1, H = L1 / 2 + 1;
+  if (!c->d_dn && !alloc_dense(c)) return TCSEM_OK;
   DenseOp &d = c->dn;
-  DenseBuild b{};
   d.kf32 = c->up_tiled && c->prec == 32;
-  d.ldax = b.ldax = (2 * H + 31) / 32 * 32;
-  d.ldb = b.ldb = (L + 1 + 15) / 16 * 16;
-  d.MP = (M + 1 + 31) / 32 * 32;
+  const DenseSizes z = dense_sizes(c, d.kf32 != 0);
+  DenseBuild b{};
+  d.ldax = b.ldax = z.ldax;
+  d.ldb = b.ldb = z.ldb;
+  d.MP = z.MP;
   d.sP = (long long)2 * H * d.MP;
-  const int ne = (M + 1) / 2, no = M / 2;
-  d.kstride = b.kstride = (long long)ne * (ne + (M + 1) / 2) + (long long)no * (no + M / 2 + 1);
-  b.Hy = M1 / 2 + 1;
-  b.ldy = (M / 2 + 1 + 31) / 32 * 32;
-  const size_t nax = (size_t)(L + 15) / 16 * 16 * d.ldax, nb = (size_t)(2 * H + 3) / 4 * 4 * d.ldb;
-  const size_t ntab = nax + 2 * nb + 2 * (size_t)(M / 2 + 1) + H;
-  const size_t kb = (size_t)H * d.kstride * (d.kf32 ? 4 : 8);
-  c->dn_bytes = ntab * 8 + kb;
-  if (hipMalloc(&c->d_dn, c->dn_bytes) != hipSuccess)
-    return fail(TCSEM_ENOMEM, "air operators: %zu bytes", c->dn_bytes);
+  d.kstride = b.kstride = z.kstride;
+  b.Hy = z.Hy;
+  b.ldy = z.ldy;
   double *p = (double *)c->d_dn;
   d.ax = b.ax = p;
-  d.bx = b.bx = p + nax;
-  d.by = b.by = b.bx + nb;
-  b.nt = b.by + nb;
+  d.bx = b.bx = p + z.nax;
+  d.by = b.by = b.bx + z.nb;
+  b.nt = b.by + z.nb;
   b.ns = b.nt + (M / 2 + 1);
   b.ng = b.ns + (M / 2 + 1);
   d.nt = M1 % 2 == 0 ? b.nt : nullptr;
   d.ns = b.ns;
   d.ng = b.ng;
-  d.kop = b.kop = p + ntab;
+  d.kop = b.kop = p + z.ntab;
   const tcsem_setup &s = c->setup;
   b.dzdx = s.dzmin / s.dxmin;
   b.dzdy = s.dzmin / s.dymin;
   b.rxy = s.dxmin / s.dymin;
   b.ryx = s.dymin / s.dxmin;
-  std::vector<double> trig(2 * (size_t)L1 + 4 * (size_t)M1);
+  std::vector<double> trig(z.ntrig);
   for (int q = 0; q < L1; ++q) {
     trig[2 * q] = std::cos(2 * kPi * q / L1);
     trig[2 * q + 1] = std::sin(2 * kPi * q / L1);
@@ -2979,45 +3032,79 @@ int build_dense(tcsem_ctx *c) {
     trig[2 * (L1 + q)] = std::cos(kPi * q / M1);
     trig[2 * (L1 + q) + 1] = std::sin(kPi * q / M1);
   }
-  const size_t ny = (size_t)b.Hy * b.ldy, ng = (size_t)H * b.Hy, ntmp = trig.size() + 6 * ny + 2 * ng;
-  double *t = nullptr;
-  auto drop = [&](int code) {
-    (void)hipFree(c->d_dn);
-    c->d_dn = nullptr;
-    return code;
-  };
-  if (hipMalloc((void **)&t, ntmp * 8) != hipSuccess)
-    return drop(fail(TCSEM_ENOMEM, "air operator tables: %zu bytes", ntmp * 8));
+  double *t = c->d_dnt;
   b.tx = (const double2 *)t;
   b.ty = b.tx + L1;
-  b.cw = t + trig.size();
-  b.sw = b.cw + ny;
-  b.cs = b.sw + ny;
-  b.ss = b.cs + ny;
-  b.ce = b.ss + ny;
-  b.se = b.ce + ny;
-  b.gx = b.se + ny;
-  b.gy = b.gx + ng;
-  hipError_t e = hipMemcpy(t, trig.data(), trig.size() * 8, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = launch_fill_zero(c->d_dn, ntab * 8, c->stream);
-  if (e == hipSuccess) e = launch_fill_zero(b.cw, (6 * ny + 2 * ng) * 8, c->stream);
+  b.cw = t + z.ntrig;
+  b.sw = b.cw + z.ny;
+  b.cs = b.sw + z.ny;
+  b.ss = b.cs + z.ny;
+  b.ce = b.ss + z.ny;
+  b.se = b.ce + z.ny;
+  b.gx = b.se + z.ny;
+  b.gy = b.gx + z.ng;
+  hipError_t e = hipMemcpy(t, trig.data(), z.ntrig * 8, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = launch_fill_zero(c->d_dn, z.ntab * 8, c->stream);
+  if (e == hipSuccess) e = launch_fill_zero(b.cw, (6 * z.ny + 2 * z.ng) * 8, c->stream);
   if (e == hipSuccess) e = launch_dense_build(b, upcont_args<double>(c), d.kf32 != 0, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  (void)hipFree(t);
-  if (e != hipSuccess) return drop(fail(TCSEM_EDEVICE, "air operators: %s", hipGetErrorString(e)));
+  (void)hipFree(c->d_dnt);
+  c->d_dnt = nullptr;
+  if (e != hipSuccess) {
+    (void)hipFree(c->d_dn);
+    c->d_dn = nullptr;
+    return fail(TCSEM_EDEVICE, "air operators: %s", hipGetErrorString(e));
+  }
   d.on = c->up_dense;
   return TCSEM_OK;
 }
 
-// Builds the operators of a context in use, where it has none.
+// Builds the operators of a context in use, where it has none and there is room.
 int ensure_dense(tcsem_ctx *c) {
-  if (c->d_dn) return TCSEM_OK;
+  if (c->dn.on) return TCSEM_OK;
   int rc = build_dense(c);
   if (!rc) rc = reserve_work(c);
   if (rc) return rc;
   c->up64 = upcont_args<double>(c);
   c->up32 = upcont_args<float>(c);
   return TCSEM_OK;
+}
+
+// Wavenumber gains of the FFT chains on the half spectrum (UpContinuation_gpu.cu:113-164); transposed, the bins that a
+// real inverse drops set to zero, for the tiled chain.
+void chain_gains(tcsem_ctx *c) {
+  const tcsem_setup *s = &c->setup;
+  const int L1 = c->g.info.L1, M1 = c->g.info.M1, H = L1 / 2 + 1;
+  c->gx.assign((size_t)M1 * H, 0.0);
+  c->gy.assign((size_t)M1 * H, 0.0);
+  const double dzdx = s->dzmin / s->dxmin, dzdy = s->dzmin / s->dymin;
+  const double rxy = s->dxmin / s->dymin, ryx = s->dymin / s->dxmin;
+  for (int iy = 0; iy < M1; ++iy)
+    for (int ix = 0; ix < H; ++ix) {
+      const double v1 = (iy < M1 / 2 + 1) ? (1.0 * kPi * iy) / M1 * dzdy : -(1.0 * kPi * (M1 - iy)) / M1 * dzdy;
+      const double u1 = (1.0 * kPi * ix) / L1 * dzdx;
+      double gxv = 1.0, gyv = 1.0;
+      if (!(ix == 0 && iy == 0)) {
+        const double rr = u1 * u1 + v1 * v1;
+        const double upcc = std::exp(-std::sqrt(rr)) * (1.0 / std::sqrt(rr));
+        gxv = rxy * u1 * upcc;
+        gyv = ryx * v1 * upcc;
+      }
+      c->gx[(size_t)iy * H + ix] = gxv;
+      c->gy[(size_t)iy * H + ix] = gyv;
+    }
+  if (!c->up_tiled) return;
+  c->gxT.assign((size_t)H * M1, 0.0);
+  c->gyT.assign((size_t)H * M1, 0.0);
+  for (int ky = 0; ky < M1; ++ky)
+    for (int kx = 0; kx < H; ++kx) {
+      double gxv = c->gx[(size_t)ky * H + kx], gyv = c->gy[(size_t)ky * H + kx];
+      if (kx == 0 && ky == 0) gxv = gyv = 0.0;
+      if (L1 % 2 == 0 && 2 * kx == L1) gxv = 0.0;
+      if (M1 % 2 == 0 && 2 * ky == M1 && (kx == 0 || (L1 % 2 == 0 && 2 * kx == L1))) gyv = 0.0;
+      c->gxT[(size_t)kx * M1 + ky] = gxv;
+      c->gyT[(size_t)kx * M1 + ky] = gyv;
+    }
 }
 
 // The form of a batch's air boundary, one for all members: two sets of launches, each member in the form that it takes
@@ -3035,8 +3122,10 @@ int batch_air(tcsem_batch *b) {
     bm += c->dn.bm;
   }
   if (!may || !(always || dense_line(b->prec == 32, kb, w, bm))) return TCSEM_OK;
-  for (tcsem_ctx *c : b->m)
+  for (tcsem_ctx *c : b->m) {
     if (int rc = ensure_dense(c)) return rc;
+    if (!c->dn.on) return TCSEM_OK;
+  }
   b->air_mat = true;
   return TCSEM_OK;
 }
@@ -3107,7 +3196,6 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
     spline_weights(c->n3, g.dy.data(), g.Y.data(), aY, g.Yn.data(), idr.data(), c->wf);
     for (int p = 0; p < aY; ++p) idr[p] = g.yN2o[aY + Ny + p] - oy;
     spline_weights(c->n3, g.dy.data() + oy, g.Y.data() + oy, aY, g.Yn.data() + aY + Ny, idr.data(), c->wb);
-    // wavenumber gains on the half spectrum (UpContinuation_gpu.cu:113-164)
     const int L1 = I.L1, M1 = I.M1, H = L1 / 2 + 1;
     make_plan(L1, c->plx);
     make_plan(M1, c->ply);
@@ -3117,27 +3205,6 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
     const bool want_lines = chain && std::strcmp(chain, "lines") == 0;
     c->up_tiled = !want_lines && c->plx.m <= 2048 && c->ply.m <= 2048 && L <= c->plx.m + 2 && M <= c->ply.m + 2;
     c->up_dense = want_lines ? 0 : choose_air(c, chain);
-    const bool chains = c->up_tiled || !c->up_dense;  // whether an FFT chain may run: its gains
-    if (chains) {
-      c->gx.assign((size_t)M1 * H, 0.0);
-      c->gy.assign((size_t)M1 * H, 0.0);
-      const double dzdx = s->dzmin / s->dxmin, dzdy = s->dzmin / s->dymin;
-      const double rxy = s->dxmin / s->dymin, ryx = s->dymin / s->dxmin;
-      for (int iy = 0; iy < M1; ++iy)
-        for (int ix = 0; ix < H; ++ix) {
-          const double v1 = (iy < M1 / 2 + 1) ? (1.0 * kPi * iy) / M1 * dzdy : -(1.0 * kPi * (M1 - iy)) / M1 * dzdy;
-          const double u1 = (1.0 * kPi * ix) / L1 * dzdx;
-          double gxv = 1.0, gyv = 1.0;
-          if (!(ix == 0 && iy == 0)) {
-            const double rr = u1 * u1 + v1 * v1;
-            const double upcc = std::exp(-std::sqrt(rr)) * (1.0 / std::sqrt(rr));
-            gxv = rxy * u1 * upcc;
-            gyv = ryx * v1 * upcc;
-          }
-          c->gx[(size_t)iy * H + ix] = gxv;
-          c->gy[(size_t)iy * H + ix] = gyv;
-        }
-    }
     if (c->up_tiled) {
       // pitches are whole 128-byte lines and avoid multiples of 1 KiB (HBM channel spread)
       auto pitch = [](int n, int per_line) {
@@ -3158,17 +3225,6 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
       c->sA = slot_stride(H * (long long)c->MA);       // complex entries
       c->sG = slot_stride(2LL * H * c->MG);            // complex entries
       c->sX = slot_stride((long long)M1 * c->XR);      // reals
-      c->gxT.assign((size_t)H * M1, 0.0);
-      c->gyT.assign((size_t)H * M1, 0.0);
-      for (int ky = 0; ky < M1; ++ky)
-        for (int kx = 0; kx < H; ++kx) {
-          double gxv = c->gx[(size_t)ky * H + kx], gyv = c->gy[(size_t)ky * H + kx];
-          if (kx == 0 && ky == 0) gxv = gyv = 0.0;
-          if (L1 % 2 == 0 && 2 * kx == L1) gxv = 0.0;
-          if (M1 % 2 == 0 && 2 * ky == M1 && (kx == 0 || (L1 % 2 == 0 && 2 * kx == L1))) gyv = 0.0;
-          c->gxT[(size_t)kx * M1 + ky] = gxv;
-          c->gyT[(size_t)kx * M1 + ky] = gyv;
-        }
     }
   }
   const size_t lds_max = 160 * 1024 - 1024;
@@ -3207,6 +3263,9 @@ int tcsem_create(const tcsem_setup *s, const double *cond, int precision, tcsem_
     tcsem_destroy(c);
     return fail(TCSEM_EDEVICE, "event record failed");
   }
+  // where the matrix form stands in for the line chain its memory decides now; a chain that may run gets its gains
+  if (c->up_dense && !c->up_tiled) (void)alloc_dense(c);
+  if (c->up_tiled || !c->up_dense) chain_gains(c);
   // device constants
   auto bail = [&](int code) {
     tcsem_destroy(c);
@@ -3377,6 +3436,7 @@ void tcsem_destroy(tcsem_ctx *c) {
   (void)hipFree(c->d_up);
   (void)hipFree(c->d_work);
   (void)hipFree(c->d_dn);
+  (void)hipFree(c->d_dnt);
   (void)hipFree(c->d_scratch);
   (void)hipFree(c->d_rx);
   (void)hipFree(c->d_rxi);
@@ -3475,7 +3535,7 @@ int tcsem_set_transmitters(tcsem_ctx *c, const tcsem_tx *tx, int ntx) {
 int tcsem_reserve_batch(tcsem_ctx *c, int nbatch) {
   if (check_ctx(c) || nbatch < 1) return fail(TCSEM_EINVAL, "bad batch size");
   int rc = TCSEM_OK;
-  if (!c->d_dn && wants_dense(c, nbatch) && (rc = build_dense(c))) return rc;
+  if (!c->dn.on && wants_dense(c, nbatch) && (rc = build_dense(c))) return rc;
   if ((rc = alloc_slots(c, nbatch))) return rc;
   c->up64 = upcont_args<double>(c);
   c->up32 = upcont_args<float>(c);
@@ -4154,7 +4214,7 @@ long tcsem_graph_replays(const tcsem_ctx *c) { return c ? c->graph_replays : -1;
 int tcsem_air_form(const tcsem_ctx *c, int nslot, size_t *bytes) {
   if (check_ctx(c)) return TCSEM_EINVAL;
   if (nslot < 1) return fail(TCSEM_EINVAL, "at least one slot");
-  if (bytes) *bytes = c->d_dn ? c->dn_bytes : 0;
+  if (bytes) *bytes = c->dn.on ? c->dn_bytes : 0;
   if (wants_dense(c, nslot)) return TCSEM_AIR_MATRIX;
   return c->up_tiled ? TCSEM_AIR_FFT : TCSEM_AIR_LINES;
 }

@@ -116,6 +116,17 @@ def test_operators_are_built_where_they_are_used(monkeypatch):
         assert np.any(a) and np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("precision,tol", [(T.FP64, 1e-11), (T.FP32, 2e-5)])
+@pytest.mark.parametrize("chain", ["", "dense"])
+@pytest.mark.parametrize("kw,form", [({}, "fft"), (BLUESTEIN, "fft"), (LONG_X, "lines"), (LONG_Y, "lines")])
+def test_no_room_for_operators(kw, form, chain, precision, tol, monkeypatch):
+    """Where device memory leaves no room for the row operators (here: more is to stay free than the card has), a
+    context is created all the same and runs its FFT chain."""
+    monkeypatch.setenv("TCSEM_UPCONT_CHAIN", chain)
+    monkeypatch.setenv("TCSEM_SPARE_MB", "1e9")
+    _plane(kw, precision, form, tol)
+
+
 TXS = [dict(B.TX, x=x, txid=q + 1) for q, x in enumerate((0.0, -100.0, 120.0, 60.0))]
 COND = B.CONDS[0]
 _REF = {}
@@ -247,6 +258,28 @@ def test_batch_form(sides, form, precision, tol, rows):
         again = [c.run(0, 1, max_steps=300)[0] for c in cx]  # a member keeps its own form, operators or not
         for a, g in zip(alone, again):
             assert np.array_equal(a, g)
+    finally:
+        for c in cx:
+            c.close()
+
+
+def test_batch_without_room_for_a_member_s_operators(monkeypatch):
+    cx = []
+    try:
+        for q, n in enumerate((256, 100, 100)):  # a batch in matrix form, above
+            st = _marine(n, 24)
+            gi = T.grid_info(st)
+            cx.append(T.Context(st, np.ones((gi.N, gi.M, gi.L)), T.FP64))
+            cx[-1].set_receivers(B._rt(T), B.RX)
+            cx[-1].set_transmitters([T.make_tx(**B.TX)])
+            cx[-1].set_pairs(8)
+        alone = [c.run(0, 1, max_steps=100)[0] for c in cx]
+        monkeypatch.setenv("TCSEM_SPARE_MB", "1e9")
+        with T.Batch(cx) as b:
+            assert b.air_form() == "fft"
+            got = b.run(max_steps=100)
+        for a, g in zip(alone, got):
+            assert np.all(decks.trace_error(g, a) < 1e-11)
     finally:
         for c in cx:
             c.close()
