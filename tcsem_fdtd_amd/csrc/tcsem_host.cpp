@@ -509,6 +509,7 @@ struct tcsem_ctx {
   // first used; only levels 0 .. 2 are written)
   int pair_by = 0, pair_pf = 1, pair_ntx = 0, pair_nty = 0, pair_nper = 0;
   int pair_set = -1, pair_set_pf = 1;  // tcsem_set_pairs' choice (-1: none), over any other
+  bool pair_asked = false;             // pairs by the caller's choice: their memory is no option
   int tune_pair_by = 0, tune_pair_pf = 1;  // the autotuner's, for its batch size tune_nbatch
   char *d_mid = nullptr;
   long pairs_done = 0;
@@ -674,11 +675,13 @@ void choose_tiling(tcsem_ctx *c, int nbatch) {
     pby = c->tune_pair_by;
     ppf = c->tune_pair_pf;
   }
+  c->pair_asked = c->pair_set >= 0;
   if (const char *e = std::getenv("TCSEM_MARCH_PAIRS")) {
     int r = 0, q = 1;
     if (std::sscanf(e, "%d,%d", &r, &q) >= 1 && (r == 0 || (pair_rows_supported(c->prec, r) && q >= 1 && q <= 2))) {
       pby = r;
       ppf = q;
+      c->pair_asked = true;
     } else {
       std::fprintf(stderr, "tcsem: TCSEM_MARCH_PAIRS=%s is not 0 or rows,pf (rows 8, 10, 12, 14, 16 (FP64: 8, 10, 11, 12); pf 1, 2)\n", e);
     }
@@ -1642,10 +1645,11 @@ bool pair_ok(tcsem_ctx *c, long room) {
   return c->pair_by > 0 && room >= 2 && c->g.info.N >= 6 && !events_ahead(c, 1);
 }
 
-hipError_t ensure_mid(tcsem_ctx *c) {
+// The intermediate state of pairs; asked: the caller chose them (an option of the library's otherwise).
+hipError_t ensure_mid(tcsem_ctx *c, bool asked) {
   if (c->d_mid) return hipSuccess;
   const size_t mb = (size_t)5 * c->nslots * c->fstride * c->esz;
-  hipError_t e = hipMalloc(&c->d_mid, mb);
+  hipError_t e = asked ? hipMalloc(&c->d_mid, mb) : optional_malloc((void **)&c->d_mid, mb, 1);
   if (e != hipSuccess) {
     c->d_mid = nullptr;
     return e;
@@ -1664,7 +1668,7 @@ hipError_t enqueue_pair(tcsem_ctx *c, const MarchArgs<T> &a, const MarchArgs<T> 
   hipStream_t st = c->stream, st2 = c->stream2;
   const UpcontArgs<T> &u = up_of<T>(c);
   hipError_t e;
-  if ((e = ensure_mid(c)) != hipSuccess) return e;
+  if ((e = ensure_mid(c, true)) != hipSuccess) return e;
   const long long org = c->PX + c->xm, fs = c->fstride * c->nslots, ps = c->pstride * c->nslots;
   T *fm = (T *)c->d_mid, *pl = (T *)c->d_planes;
   PairArgs<T> p{};
@@ -1794,8 +1798,11 @@ int advance(tcsem_ctx *c, long room) {
     return rc ? rc : c->graph_k;
   }
   if (pair_ok(c, room)) {
-    const int rc = do_pair<T>(c);
-    return rc ? rc : 2;
+    if (c->pair_asked || ensure_mid(c, false) == hipSuccess) {
+      const int rc = do_pair<T>(c);
+      return rc ? rc : 2;
+    }
+    c->pair_by = 0;  // no room for the intermediate state: this run takes one step at a time
   }
   const int rc = do_step<T>(c);
   return rc ? rc : 1;
@@ -2055,6 +2062,7 @@ struct tcsem_batch {
   size_t pwork_cap = 0;
   int pwork_len = 0;
   long pairs_done = 0;
+  bool pair_full = false;  // no room for the members' intermediate states
   bool air_mat = false;  // the air boundary of every member in matrix form (batch_air)
 };
 
@@ -2214,7 +2222,7 @@ int batch_records(tcsem_batch *b, int by, int pf, MarchArgs<T> &la, UpcontArgs<T
     std::vector<int> tiles(nm);
     for (int q = 0; q < nm; ++q) {
       tcsem_ctx *c = b->m[q];
-      HIPCHK(ensure_mid(c));
+      HIPCHK(ensure_mid(c, true));
       HIPCHK(hipStreamSynchronize(c->stream));
       const long long org = c->PX + c->xm, fs = c->fstride * c->nslots, ps = c->pstride * c->nslots;
       T *fm = (T *)c->d_mid, *pl = (T *)c->d_planes;
@@ -2448,13 +2456,16 @@ bool batch_pair_ok(tcsem_batch *b) {
 
 // Rows of the batch's two-step passes: tcsem_batch_set_pairs' choice, else TCSEM_MARCH_PAIRS
 // ("0" or "rows[,1]"), else the autotuner's, else pass_rows over the members' tiles (0: one step at a time).
-int batch_pair_rows(tcsem_batch *b) {
+int batch_pair_rows(tcsem_batch *b, bool &asked) {
+  asked = true;
   if (b->pair_set >= 0) return b->pair_set;
   if (const char *e = std::getenv("TCSEM_MARCH_PAIRS")) {
     int r = 0, q = 1;
     if (std::sscanf(e, "%d,%d", &r, &q) >= 1 && (r == 0 || (pair_rows_supported(b->prec, r) && q == 1))) return r;
   }
+  asked = false;
   if (b->pair_tuned >= 0) return b->pair_tuned;
+  if (b->pair_full) return 0;
   auto tiles = [&](int rows) {
     long long n = 0;
     for (size_t q = 0; q < b->m.size(); ++q)
@@ -2469,6 +2480,27 @@ int batch_pair_rows(tcsem_batch *b) {
       mb += 10.0 * I.L * I.M * I.N * (b->prec / 8) * 1e-6;
     }
   return pass_rows(b->prec, tiles, mb, device_cus());
+}
+
+// Every member's intermediate state, or none where there is no room for all; the batch then stays with one step at
+// a time.
+bool batch_mid(tcsem_batch *b) {
+  std::vector<tcsem_ctx *> got;
+  for (tcsem_ctx *c : b->m) {
+    if (c->d_mid) continue;
+    if (ensure_mid(c, false) == hipSuccess) {
+      got.push_back(c);
+      continue;
+    }
+    for (tcsem_ctx *g : got) {
+      (void)hipStreamSynchronize(g->stream);
+      (void)hipFree(g->d_mid);
+      g->d_mid = nullptr;
+    }
+    b->pair_full = true;
+    return false;
+  }
+  return true;
 }
 
 // Orders the batch's work before what is issued next on the batch's and the members' streams.
@@ -2538,7 +2570,9 @@ int batch_step_t(tcsem_batch *b, int nsteps) {
   batch_tiling(b, by, pf);
   MarchArgs<T> la;
   UpcontArgs<T> ul;
-  const int pby = nsteps >= 2 ? batch_pair_rows(b) : 0;
+  bool asked = false;
+  int pby = nsteps >= 2 ? batch_pair_rows(b, asked) : 0;
+  if (pby && !asked && !batch_mid(b)) pby = 0;
   if (int rc = batch_records<T>(b, by, pf, la, ul, pby)) return rc;
   // the record parity flips once per step or pair (a pair leaves its result where one step would)
   int par = 0;
@@ -4064,6 +4098,7 @@ int tcsem_set_pairs(tcsem_ctx *c, int rows, int pf) {
   if (rows && c->g.info.N < 6) return fail(TCSEM_EINVAL, "two-step pass needs at least 6 levels");
   c->pair_set = rows;
   c->pair_set_pf = pf;
+  c->pair_asked = true;
   pair_tiling(c, rows, pf);
   return TCSEM_OK;
 }
