@@ -596,12 +596,12 @@ void pair_tiling(tcsem_ctx *c, int by, int pf) {
 // (320) 20.7 / 19.6; FP64 120 x 120 x 160 (90) 15.4 / 18.6, 140 x 140 x 120 (105) 23.4 / 21.0, 256 x 256 x
 // 160 43.3 / 30.0.
 template <typename F>
-int pass_rows(int prec, F &&tiles, double state_mb, int cu) {
+int pass_rows(int prec, F &&tiles, double state_mb, int levels, int cu) {
   if (2 * tiles(8) < (prec == 32 ? 256 : 200) * (long long)cu / 256) return 0;
   int best = 0;
   double cost = 1e300;
   for (int b : {8, 10, 11, 12, 14, 16}) {
-    if (!pair_rows_supported(prec, b)) continue;
+    if (!pair_rows_supported(prec, b) || !pass_fits(prec / 8, b, levels)) continue;
     const long long rounds = (tiles(b) + cu - 1) / cu;
     double w = b;
     if (state_mb > 256.0)
@@ -670,7 +670,7 @@ void choose_tiling(tcsem_ctx *c, int nbatch) {
   int ppf = 2;
   int pby = pass_rows(
       c->prec, [&](int b) { return (long long)pass_tiles_x(c->prec, b, L) * pass_tiles_y(M, b) * nbatch; },
-      10.0 * L * M * N * nbatch * c->esz * 1e-6, cu);
+      10.0 * L * M * N * nbatch * c->esz * 1e-6, N, cu);
   if (c->tune_nbatch == nbatch) {
     pby = c->tune_pair_by;
     ppf = c->tune_pair_pf;
@@ -1988,7 +1988,7 @@ int autotune_pairs(tcsem_ctx *c, int nbatch, int nsteps, int *best_by, int *best
   std::vector<Shape> shapes;
   for (int by : {12, 14, 16, 11, 10, 8})
     for (int pf = 1; pf <= 2; ++pf)
-      if (pair_rows_supported(c->prec, by)) shapes.push_back({by, pf, 1e300});
+      if (pair_rows_supported(c->prec, by) && pass_fits(c->esz, by, c->g.info.N)) shapes.push_back({by, pf, 1e300});
   for (int round = 0; round < 2 && rc == TCSEM_OK; ++round)
     for (Shape &sh : shapes) {
       const int by = sh.by, pf = sh.pf;
@@ -2474,12 +2474,14 @@ int batch_pair_rows(tcsem_batch *b, bool &asked) {
     return n;
   };
   double mb = 0.0;
+  int levels = 0;  // the launch's LDS holds the deepest member's coefficients, finished or not
+  for (size_t q = 0; q < b->m.size(); ++q) levels = std::max(levels, b->m[q]->g.info.N);
   for (size_t q = 0; q < b->m.size(); ++q)
     if (b->active[q]) {
       const tcsem_grid_info &I = b->m[q]->g.info;
       mb += 10.0 * I.L * I.M * I.N * (b->prec / 8) * 1e-6;
     }
-  return pass_rows(b->prec, tiles, mb, device_cus());
+  return pass_rows(b->prec, tiles, mb, levels, device_cus());
 }
 
 // Every member's intermediate state, or none where there is no room for all; the batch then stays with one step at
@@ -2665,7 +2667,11 @@ int batch_autotune_t(tcsem_batch *b, int nsteps, int *best_by, int *best_pf, int
       const hipError_t e = hipMemcpy(b->d_scal, scal2.data(), scal2.size() * sizeof(double), hipMemcpyHostToDevice);
       if (e != hipSuccess) rc = fail(TCSEM_EDEVICE, "batch autotune: %s", hipGetErrorString(e));
     }
-    const std::vector<int> prow = b->prec == 64 ? std::vector<int>{12, 11, 10, 8} : std::vector<int>{12, 14, 16, 10, 8};
+    std::vector<int> prow;
+    int levels = 0;
+    for (const tcsem_ctx *c : b->m) levels = std::max(levels, c->g.info.N);
+    for (int r : {12, 14, 16, 11, 10, 8})
+      if (pair_rows_supported(b->prec, r) && pass_fits(b->prec / 8, r, levels)) prow.push_back(r);
     const int npair = std::max(1, nsteps / 2);
     // two interleaved rounds over the pass heights; each keeps its faster time
     std::vector<double> pm(prow.size(), 1e300);

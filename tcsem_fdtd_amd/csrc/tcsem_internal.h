@@ -43,6 +43,12 @@ constexpr int pass_cols(int esz, int rows) {
   return esz == 8 || rows == 12 ? 56 : rows == 16 ? 48 : 60;
 }
 
+// Whether a pass of that many rows fits a compute unit's 160 KB of LDS at N levels: 14 tile planes, the table of the
+// conductivity index, three coefficients a level (FP64 12 rows: up to 3157 levels, 11 3456, 10 3754).
+constexpr bool pass_fits(int esz, int rows, int levels) {
+  return (14LL * rows * kMarchLanes + 256 + 3LL * levels) * esz <= 160 * 1024;
+}
+
 // One injected E cell: E[comp](k, j, i) -= amp * w each source step (ElectricalFiled.cu:347-475).
 // The same record lists the B cells a source step recomputes (comp 3 Bx, 4 By; w unused).
 struct SrcCell {
