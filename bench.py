@@ -275,17 +275,28 @@ def roofline(res, esz, nbatch, traffic_entry):
             "span": "per step: the lower and the top launch of k_march, the lower one from the start of its k_zsum pass when the tiling runs one"}
 
 
-def traffic_key(key, res):
-    """The counter summary's key for a run: the two-step pass has entries of its own, one per pass
-    shape where that shape was counted (key_pairs_rows,pf), else one for the workload."""
-    pr = res.get("pairs")
-    if not pr:
-        return key
-    if pr.get("pf"):
-        exact = "%s_pairs_%d,%d" % (key, pr["rows"], pr["pf"])
-        if load_traffic(exact)[0] is not None:
-            return exact
-    return key + "_pairs"
+def shape_of(res):
+    """The march shape of a run as the counter summary writes it: "rows,pf" of the two-step pass ("rows" for a model
+    batch's), else the one-step tiling; None where the library's heuristic picked that."""
+    pr, t = res.get("pairs"), res.get("tiling")
+    if pr:
+        return "%d,%d" % (pr["rows"], pr["pf"]) if pr.get("pf") else "%d" % pr["rows"]
+    if not t:
+        return None
+    if "zchunks" not in t:
+        return "%d,%d" % (t["rows"], t["pf"])
+    return "%d,%d,%d,%s,%d" % (t["rows"], t["pf"], t["zchunks"], t["zsum"], t["sigma8"])
+
+
+def counted_traffic(key, res):
+    """(HBM bytes, shape) that the counter summary holds for the shape that ran, (None, None) where it holds another's."""
+    shape = shape_of(res)
+    keys = ["%s_pairs_%s" % (key, shape), key + "_pairs"] if res.get("pairs") else [key]
+    for k in keys:
+        got = load_traffic(k)
+        if got[0] is not None and got[1] == shape:
+            return got
+    return None, None
 
 
 def _fft_len(n):
@@ -536,8 +547,8 @@ def accuracy(T, W):
 
 
 def load_traffic(key):
-    """HBM bytes per step of k_march from the committed counter summary (profiles/traffic.json),
-    with the march tiling they were counted for; (None, None) when absent."""
+    """HBM bytes per step of k_march, or per launch of the two-step pass, from the committed counter summary
+    (profiles/traffic.json), with the shape they were counted for; (None, None) when absent."""
     p = os.path.join(ROOT, "profiles", "traffic.json")
     try:
         with open(p) as f:
@@ -625,22 +636,22 @@ def main():
         "config": {"workload": "large_5 512x512x256, 1024x1024 air plane, x-dipole 1 of 3, 401 receivers, FP32 fields",
                    "cells": rl32["L"] * rl32["M"] * rl32["N"], "batch": 1, "parallelism": "single GPU",
                    "march_tiling": rl32["tiling"]},
-        "roofline": roofline(rl32, 4, 1, load_traffic(traffic_key("large_5_fp32", rl32))),
+        "roofline": roofline(rl32, 4, 1, counted_traffic("large_5_fp32", rl32)),
         "kernel_ms": kern(rl32),
         "side_kernels": side_kernels(rl32, big, 4, 1),
         "fp64_single": {"workload": "large_5 512x512x256, FP64 fields, the same window",
                         "value": round(rl64["gcell_s"], 3), "ms_per_step": round(rl64["ms_per_step"], 5),
-                        "roofline": roofline(rl64, 8, 1, load_traffic(traffic_key("large_5_fp64", rl64))),
+                        "roofline": roofline(rl64, 8, 1, counted_traffic("large_5_fp64", rl64)),
                         "march_tiling": rl64["tiling"], "kernel_ms": kern(rl64),
                         "fp32_vs_fp64_ex_rel_l2_after_window": big_err},
         "marine_3d": {"workload": "marine_3d 256x256x160, 512x512 air plane, 1 x-dipole, 101 receivers",
                       "steps": args.steps, "warmup": args.warmup,
                       "fp32": {"value": round(r32["gcell_s"], 3), "ms_per_step": round(r32["ms_per_step"], 5),
-                               "roofline": roofline(r32, 4, 1, load_traffic(traffic_key("marine_3d_fp32", r32))),
+                               "roofline": roofline(r32, 4, 1, counted_traffic("marine_3d_fp32", r32)),
                                "march_tiling": r32["tiling"], "kernel_ms": kern(r32),
                                "side_kernels": side_kernels(r32, deck, 4, 1)},
                       "fp64": {"value": round(r64["gcell_s"], 3), "ms_per_step": round(r64["ms_per_step"], 5),
-                               "roofline": roofline(r64, 8, 1, load_traffic(traffic_key("marine_3d_fp64", r64))),
+                               "roofline": roofline(r64, 8, 1, counted_traffic("marine_3d_fp64", r64)),
                                "march_tiling": r64["tiling"], "kernel_ms": kern(r64),
                                "one_step": r64["one_step"]},
                       "fp32_vs_fp64_ex_rel_l2_after_window": field_err},
@@ -648,18 +659,18 @@ def main():
                          "workload": "towline %d x-dipoles, marine_3d grid" % args.batch,
                          "steps": nb, "warmup": args.warmup,
                          "ms_per_step": round(rb["ms_per_step"], 5),
-                         "roofline": roofline(rb, 4, args.batch, load_traffic(traffic_key("towline32_fp32", rb))),
+                         "roofline": roofline(rb, 4, args.batch, counted_traffic("towline32_fp32", rb)),
                          "march_tiling": rb["tiling"], "kernel_ms": kern(rb),
                          "side_kernels": side_kernels(rb, tow, 4, args.batch)},
         "uneven_models": {"workload": "64 models, grids 96^3 .. 224x224x160 (%d cells), 1 x-dipole and 41 receivers each"
                                       % m32["cells"], "steps": nm, "warmup": wm,
                           "fp32": {"value": round(m32["gcell_s"], 3), "ms_per_step": round(m32["ms_per_step"], 5),
-                                   "roofline": models_roofline(m32, 4, load_traffic(traffic_key("uneven64_fp32", m32))),
+                                   "roofline": models_roofline(m32, 4, counted_traffic("uneven64_fp32", m32)),
                                    "march_tiling": m32["tiling"], "kernel_ms": kern(m32),
                                    "unbatched": {k: round(v, 5) if isinstance(v, float) else v
                                                  for k, v in m32["unbatched"].items()}},
                           "fp64": {"value": round(m64["gcell_s"], 3), "ms_per_step": round(m64["ms_per_step"], 5),
-                                   "roofline": models_roofline(m64, 8, load_traffic(traffic_key("uneven64_fp64", m64))),
+                                   "roofline": models_roofline(m64, 8, counted_traffic("uneven64_fp64", m64)),
                                    "march_tiling": m64["tiling"],
                                    "kernel_ms": kern(m64)},
                           "fp32_vs_fp64_ex_rel_l2_after_window": models_err},
