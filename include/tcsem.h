@@ -253,13 +253,14 @@ int tcsem_air_form(const tcsem_ctx *ctx, int nslot, size_t *bytes);
 
 /* Two steps per lower pass (no counterpart in the reference, whose steps each read and write
  * the whole state): with rows 8, 10, 12, 14 or 16 (FP64: 8, 10, 11 or 12; workgroup rows of the pass) and pf 1 or 2 (prefetch
- * depth), tcsem_step and tcsem_run take each two consecutive steps after the source wavelet
+ * depth), tcsem_step and tcsem_run take each two consecutive steps, those of the source wavelet too,
  * whose first holds no receiver sample as one pass over levels N-1 .. 3 of both steps (the
  * intermediate state stays on chip there), then the top levels of each step as usual.  The
  * results equal, bit for bit, those of one step at a time with an unchunked march (tested).
  * rows 0 turns it off.  Without a call the library decides at tcsem_begin: TCSEM_MARCH_PAIRS ("0"
  * or "rows,pf"), else the autotuner's choice for the batch size, else, where 8-row passes give about
- * half the CUs a workgroup, the height whose rounds of one workgroup per CU cost least (prefetch 2); a
+ * half the CUs a workgroup, the height whose rounds of one workgroup per CU cost least (prefetch 2; one step at a
+ * time where device memory has no room for the intermediate state); a
  * call holds for the context's later runs.  Graph replays, where on, take precedence.  Needs N >= 6.
  * tcsem_pair_info reports the setting and the pairs taken so far; tcsem_pair_timing the average
  * device time [ms] of the two-step pass alone (timing enabled; its top launches count in
@@ -297,8 +298,8 @@ int tcsem_batch_timing(tcsem_batch *batch, double t[3], long n[3]);
 /* Two steps per pass for the batch (no counterpart in the reference), as tcsem_set_pairs for a
  * context: rows 8, 10, 12, 14 or 16 (FP64: 8, 10, 11 or 12) at prefetch depth 1, or 0 (one step at a time), over
  * the library's choice (TCSEM_MARCH_PAIRS, the batch autotuner's pick, else as for a context over the
- * members' pass tiles).  Pairs run when every member
- * still sampling is past its source wavelet and takes no sample after the pair's first step.
+ * members' pass tiles).  Two steps, of the source wavelet too, make a pair when no member still
+ * sampling takes a sample after the first.
  * The results equal one step at a time, bit for bit (tested).  tcsem_batch_pair_info: the rows
  * of the last step call (0: one step at a time), the autotuner's pick (-1: not tuned) and the
  * pairs taken; tcsem_batch_pair_timing: the pass's average device time while timing is enabled. */

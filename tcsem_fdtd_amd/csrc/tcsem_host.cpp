@@ -586,8 +586,9 @@ void pair_tiling(tcsem_ctx *c, int by, int pf) {
 // Default height of the two-step pass for a grid, a transmitter batch or a model batch (0: one step at a
 // time); tiles(b): its workgroups at b rows, state_mb: old and new state, MB, levels: of the deepest grid.
 // A compute unit holds one workgroup of a pass, so the pass takes rounds of `cu` of them, and a round the
-// time weighed here (us per level of 512 x 512 x 256, FP32 0.87 at 16 rows; fitted to 17 FP32 and 24 FP64 grids,
-// 90 x 90 to 512 x 512, 1 to 16 slots, where the pick is within 0.2% and 1% of the fastest height on average).
+// time weighed here, in the rows that an unhindered tile would have (fitted to 17 FP32 and 24 FP64 grids, 90 x 90 to
+// 512 x 512, 1 to 16 slots, where the pick is within 0.2% and 1% of the fastest height on average; a round of 16 FP32
+// rows takes 1.4 us a level on 512 x 512 x 256: 19.0).
 // 10-row FP64 tiles weigh less alone in a round, where bandwidth is not what bounds them: 256 x 256 x 160, 10 / 11
 // rows 29.9 / 30.9 ms, against two rounds of 398 x 354 x 180, 88.5 / 86.7.  A state that stays in the 256 MB
 // memory-side cache makes the rows alone count (512 x 512 x 20, 200 steps, 8 to 16 rows: 27.6 to 28.3 ms).
@@ -870,15 +871,17 @@ UpcontArgs<T> upcont_args(tcsem_ctx *c) {
 }
 
 // Device memory that a run can do without: refused, with no error left behind, where it does not fit, where it would
-// take more than 1/share of the free memory, or where it would not leave TCSEM_SPARE_MB free.
+// take more than 1/share of the free memory, or where it would not leave TCSEM_SPARE_MB free.  A few megabytes are
+// not weighed (the query takes 0.2 ms, a tenth of what a small context takes to create).
 hipError_t optional_malloc(void **p, size_t bytes, size_t share) {
-  *p = nullptr;
   const char *e = std::getenv("TCSEM_SPARE_MB");
   const double spare = e ? std::atof(e) * 1e6 : 0.0;
-  size_t avail = 0, total = 0;
-  if (hipMemGetInfo(&avail, &total) == hipSuccess && (double)bytes * share <= (double)avail - spare &&
-      hipMalloc(p, bytes) == hipSuccess)
-    return hipSuccess;
+  bool room = bytes <= ((size_t)16 << 20) && spare <= 0.0;
+  if (!room) {
+    size_t avail = 0, total = 0;
+    room = hipMemGetInfo(&avail, &total) == hipSuccess && (double)bytes * share <= (double)avail - spare;
+  }
+  if (room && hipMalloc(p, bytes) == hipSuccess) return hipSuccess;
   (void)hipGetLastError();
   *p = nullptr;
   return hipErrorOutOfMemory;
@@ -914,14 +917,14 @@ void free_run(tcsem_ctx *c) {
   c->begun = false;
 }
 
-// Work planes of the air boundary for c->nslots slots.  Bytes per slot: tiled chain A and G (complex of the field
+// Work planes of the air boundary for nslots slots.  Bytes per slot: tiled chain A and G (complex of the field
 // type) and Bx, By (field type); line chain cplx (complex FP64), tx, bxr (also the y-padding rows), byr (FP64); the
 // matrix form 3 planes of 2 H x MP (FP64), beside the tiled chain's need (the slot count decides between them), in
 // place of the line chain's.  Called again after the operators were built: the planes may grow.
-int reserve_work(tcsem_ctx *c) {
+int reserve_work(tcsem_ctx *c, int nslots) {
   const size_t chain = c->up_tiled ? (size_t)(2 * c->sA + 2 * c->sG + 2 * c->sX) * c->esz
                                    : (c->up_dense ? 0 : (size_t)5 * c->wstride * sizeof(double));
-  const size_t wb = (size_t)c->nslots * std::max(chain, (size_t)(3 * c->dn.sP) * sizeof(double));
+  const size_t wb = (size_t)nslots * std::max(chain, (size_t)(3 * c->dn.sP) * sizeof(double));
   if (wb <= c->work_cap) return TCSEM_OK;
   drop_graphs(c);
   HIPCHK(hipStreamSynchronize(c->stream2));
@@ -935,7 +938,7 @@ int reserve_work(tcsem_ctx *c) {
 }
 
 int alloc_slots(tcsem_ctx *c, int nslots) {
-  if (nslots <= c->nslots) return reserve_work(c);
+  if (nslots <= c->nslots) return reserve_work(c, c->nslots);
   drop_graphs(c);
   HIPCHK(hipStreamSynchronize(c->stream));
   (void)hipFree(c->d_fields);
@@ -956,6 +959,7 @@ int alloc_slots(tcsem_ctx *c, int nslots) {
   const size_t pb = (size_t)7 * nslots * c->pstride * c->esz;
   if (hipMalloc(&c->d_fields, fb) != hipSuccess) return fail(TCSEM_ENOMEM, "field allocation of %zu bytes failed", fb);
   if (hipMalloc(&c->d_planes, pb) != hipSuccess) return fail(TCSEM_ENOMEM, "plane allocation failed");
+  if (const int rc = reserve_work(c, nslots)) return rc;
   const size_t zb = (size_t)(kMaxChunks - 1) * nslots * c->pstride * c->esz;
   if (hipMalloc(&c->d_zs, zb) != hipSuccess) return fail(TCSEM_ENOMEM, "chunk-sum allocation failed");
   HIPCHK(launch_fill_zero(c->d_zs, zb, c->stream));
@@ -964,10 +968,6 @@ int alloc_slots(tcsem_ctx *c, int nslots) {
   HIPCHK(hipStreamSynchronize(c->stream));
   c->nslots = nslots;
   c->cur = 0;
-  if (const int rc = reserve_work(c)) {
-    c->nslots = 0;
-    return rc;
-  }
   return TCSEM_OK;
 }
 
@@ -3103,7 +3103,7 @@ int build_dense(tcsem_ctx *c) {
 int ensure_dense(tcsem_ctx *c) {
   if (c->dn.on) return TCSEM_OK;
   int rc = build_dense(c);
-  if (!rc) rc = reserve_work(c);
+  if (!rc) rc = reserve_work(c, c->nslots);
   if (rc) return rc;
   c->up64 = upcont_args<double>(c);
   c->up32 = upcont_args<float>(c);

@@ -629,7 +629,7 @@ k_march(const MarchArgs<T> la, const MarchArgs<T> *geo) {
 // workgroup owns pass_cols columns in the middle and BY - 4 rows: step A is exact one ring further out than
 // step B (the neighbours its curls read are one cell further out still).  Cells outside the grid compute as zero,
 // as memory holds them.
-// Bound by HBM where its tiles come in several rounds (512 x 512 x 256 FP32: 3.1 GB in 0.72 ms) and by the chain
+// Bound by HBM where its tiles come in several rounds (512 x 512 x 256 FP32: 3.2 GB in 0.72 ms) and by the chain
 // of a level's phases where they come in one.  147 vector instructions per lane and level (FP32), against 210
 // with selects for the grid's edge, address arithmetic per access and the two-level delay lines moved
 // between registers: same FP32 time at the old 60-column tiles, whose shared store segments bound it, but what let
